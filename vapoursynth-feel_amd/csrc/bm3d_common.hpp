@@ -20,6 +20,45 @@ __host__ __device__ inline uint32_t entry_x(uint32_t e) { return e & 0x3FFFu; }
 __host__ __device__ inline uint32_t entry_y(uint32_t e) { return (e >> 14) & 0x3FFFu; }
 __host__ __device__ inline uint32_t entry_z(uint32_t e) { return e >> 28; }
 
+// Run of bm3d_match_cols: nb ref blocks of vb consecutive grid rows, windows of
+// at most rw x rh candidates, a source region of at most rcols x rrows pixels
+// with LDS row stride ss (an odd multiple of 4: 16-byte reads of 16 rows fall
+// on different banks), column stride hr of its sums (odd).
+struct ColsGeometry {
+    int nb, vb, rw, rh, rcols, rrows, ss, hr;
+};
+
+// Its LDS layout, as float offsets.
+struct ColsLayout {
+    int h, box, qk, keys, bounds, stage, coef, norm, over, total;
+    int xblk;  // blocks of a grid row that the exact search takes at once, in the place of h .. bounds
+};
+
+__host__ __device__ constexpr ColsLayout cols_layout(const ColsGeometry &g)
+{
+    const int blocks = g.nb * g.vb, hcols = g.rcols & ~7;  // (groups of 8 sums of rcols - 7 columns)
+    const int h = g.rrows * g.ss + 8, box = h + hcols * g.hr, qk = (box + (g.rcols - 7) * ((g.rrows - 7) | 1) + 3) & ~3;
+    // the 8-column sums of squares; after them each grid row's corr, then its
+    // keys
+    const int corr = (g.nb * 8 * (g.rh | 1) + 3) & ~3, row = g.nb * g.rw * 8, first = corr > row ? corr : row;
+    const int keys = qk + first, kend = g.vb > 1 ? keys + first : keys, qend = (qk + hcols * g.hr + 3) & ~3;
+    const int bounds = kend > qend ? kend : qend, stage = bounds + ((blocks * g.rw + 3) & ~3);
+    const int coef = stage + blocks * 32, norm = coef + blocks * 8, over = norm + blocks * 8;
+    // the exact search: staged positions, the source region, per block and
+    // window row 3 keys and 16-bit distances
+    const int per = g.rh * 3 + (g.rh * g.rw + 1) / 2, room = stage - h - 256 - g.rcols * (g.rrows | 1) - 1;
+    const int fit = room / per, xblk = fit < g.nb ? fit : g.nb;
+    return ColsLayout{h, box, qk, keys, bounds, stage, coef, norm, over, over + ((blocks + 4 + 3) & ~3), xblk};
+}
+
+// For frames at least as large as the region.
+__host__ __device__ constexpr ColsGeometry cols_geometry(int bm_range, int step, int vb)
+{
+    const int n = 2 * bm_range + 1, nb = 256 / n < 16 ? 256 / n : 16;
+    const int rcols = (nb - 1) * step + 8 + 2 * bm_range, rrows = (vb - 1) * step + 8 + 2 * bm_range;
+    return ColsGeometry{nb, vb, n, n, rcols, rrows, ((rcols + 7) & ~7) + 4, rrows | 1};
+}
+
 // Block matching: one estimate's search, for every active ref block.
 struct MatchArgs {
     const float *plane[kMaxWindow];  // search clip, window positions z = 0..2r
@@ -35,6 +74,8 @@ struct MatchArgs {
     // layout (column-major source region, per-block distance rows)
     int run_blocks, runs_x;
     int region_cols, region_rows, dist_cols;
+    // nonzero: bm3d_match_cols with runs of that many grid rows instead
+    int cols_vb;
     // temporal search after bm3d_match_rows: distance rows per wavefront
     // (ps_num * (2 ps_range + 1)) for the threshold selection, 0: list
     int t_rows;

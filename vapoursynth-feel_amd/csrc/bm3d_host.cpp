@@ -217,6 +217,7 @@ struct Instance {
     // workgroup run and the LDS layout; run_blocks == 0 selects the
     // per-wavefront search instead
     int run_blocks = 0, runs_x = 0, region_cols = 0, region_rows = 0, dist_cols = 0;
+    int cols_vb = 0;             // grid rows per run of bm3d_match_cols (0: bm3d_match_rows)
     int pred_pair = 0;           // temporal search: both directions per wavefront
     int t_rows = 0;  // temporal threshold selection: distance rows per wavefront (0: list)
     float *dst_dev = nullptr;    // one plane
@@ -614,6 +615,7 @@ struct Instance {
         m.region_cols = region_cols;
         m.region_rows = region_rows;
         m.dist_cols = dist_cols;
+        m.cols_vb = cols_vb;
         m.t_rows = t_rows;
         m.pred_pair = pred_pair;
         m.operand = operand;
@@ -1068,6 +1070,16 @@ std::string parse_args(const vsfeel_bm3d_args &a, Instance &d)
                 d.region_cols = cols;
                 d.region_rows = rh + 7;
                 d.dist_cols = dcols;
+            }
+        }
+        // bm3d_match_cols where it was compiled and the frame holds its run's
+        // region, of two grid rows where that leaves two workgroups for every
+        // compute unit
+        for (int vb = 2; vb >= 1 && d.run_blocks > 0 && d.cols_vb == 0; --vb) {
+            const ColsGeometry g = cols_geometry(16, 4, vb);
+            if (d.bm_range == 16 && d.block_step == 4 && d.width >= g.rcols && d.height >= g.rrows &&
+                (vb == 1 || (d.nx + g.nb - 1) / g.nb * ((d.ny + 1) / 2) >= 2 * kComputeUnits)) {
+                d.cols_vb = vb;
             }
         }
         if (d.run_blocks > 0 && d.radius > 0) {

@@ -3,6 +3,9 @@
 //   bm3d_match_rows       spatial search of the sliding metric (radius < 3),
 //                         a run of reference blocks per workgroup, a window
 //                         row per thread, threshold selection of the top-8
+//   bm3d_match_cols       the same for wide windows: a window column per
+//                         thread, distances expanded into sums shared by the
+//                         run, exact distances of a shortlist
 //   bm3d_match_predictive temporal predictive search after it (radius 1-2),
 //                         one wavefront per reference block, both directions
 //   bm3d_match            block matching one wavefront per reference block:
@@ -21,6 +24,8 @@
 // must be fused is written as __builtin_fmaf, everything else rounds twice,
 // which is what keeps distances, coefficients and thresholds bit-identical to
 // the CPU restatement of the reference shaders.
+
+#include <type_traits>
 
 #include "bm3d_device.hpp"
 
@@ -107,7 +112,7 @@ __device__ __forceinline__ uint3 scan_row_sliding(const float *cb, int cbs, cons
 // D(k) of one window row exactly as scan_row_sliding computes it (same
 // column SSDs, same summation tree)
 template <int CM>
-__device__ __forceinline__ float dist_at(const float *cb, const float *col0, int CS, int k)
+__device__ __forceinline__ float row_dist_at(const float *cb, const float *col0, int CS, int k)
 {
     float v[8];
 #pragma unroll
@@ -142,11 +147,10 @@ struct SpatialRows {
     __device__ uint32_t xy(int row, int k) const { return uint32_t(left + k) | (uint32_t(top + row) << 16); }
     __device__ int row_of(uint32_t xy) const { return int(xy >> 16) - top; }
     __device__ int k_of(uint32_t xy) const { return int(xy & 0xFFFFu) - left; }
-    __device__ float exact(int row, int k) const { return dist_at<CM>(cb, col0 + row, CS, k); }
+    __device__ float exact(int row, int k) const { return row_dist_at<CM>(cb, col0 + row, CS, k); }
 };
 
 constexpr int kStageBatch = 16;  // loads a lane keeps in flight while staging
-
 
 // ascending 8-entry list of one lane: insert v (the largest drops out)
 __device__ __forceinline__ void list8_insert(uint32_t (&h)[8], uint32_t v)
@@ -162,7 +166,7 @@ __device__ __forceinline__ void list8_insert(uint32_t (&h)[8], uint32_t v)
 // The 8th smallest of the values a 16-lane row holds in its lanes' ascending
 // lists h, ties counted: the smallest m with at least 8 values <= m (~0u when
 // the row holds fewer than 8).  Consumes the lists.
-__device__ __forceinline__ uint32_t row_eighth(uint32_t (&h)[8], int lane)
+__device__ __forceinline__ uint32_t lists_eighth(uint32_t (&h)[8], int lane)
 {
     const int grp = lane >> 4;
     uint32_t tk = ~0u;
@@ -233,7 +237,7 @@ __device__ int select16(const uint32_t *rt, const uint16_t *db, int dcols, int n
         list8_insert(h, rt[3 * r + 1]);
         list8_insert(h, rt[3 * r + 2]);
     }
-    thr = row_eighth(h, lane) | pm;
+    thr = lists_eighth(h, lane) | pm;
 
     // Gathers the candidates that may be at or below thr (their positions,
     // the first 16 in sxy); returns their number and the rows scanned (bit q:
@@ -321,7 +325,7 @@ __device__ int select16(const uint32_t *rt, const uint16_t *db, int dcols, int n
                 }
             }
         }
-        const uint32_t t = row_eighth(h, lane);
+        const uint32_t t = lists_eighth(h, lane);
         const bool tighter = staged > 16 && thr > 0xFFFFu && t < thr;
         if (__ballot(tighter) != 0) {
             if (tighter) {
@@ -721,6 +725,1233 @@ __global__ __launch_bounds__(256) void bm3d_match_rows(MatchArgs A)
 }
 
 // ---------------------------------------------------------------------------
+// Spatial search of the sliding metric for wide windows.  A workgroup takes a
+// run of NB consecutive ref blocks of VB consecutive grid rows; their windows
+// share one source region, staged row-major in LDS.
+//
+// The metric of candidate k of a window row, with s the source and c_j the
+// reference block's columns, is D(k) = sum_j |c_min(j-k.., 7) - s|^2 over the
+// candidate's 8 columns, which for k >= 7 all meet column 7.  Expanded,
+//   D~(k) = |R_k|^2 + box - 2 sum_i c7[i] h(cx, cy + i)
+//           - 2 sum_{j = k..6} sum_i (c_j - c7)[i] s(left + j, cy + i)
+// with box and h the 8x8 sums of s^2 and the 8-column sums of s, which every
+// block of the run shares: 8 multiply-adds per candidate instead of a column
+// SSD (23 operations) and its tree, and the last term (`corr`, with |R_k|^2)
+// once per row for the first 7 candidates.  D~ only ranks: it bounds D, and
+// the few candidates that may be among the 8 nearest get the reference's FP32
+// distance (column SSDs and summation tree), which alone decides.  All sums
+// use s - m, m the mean of a few of the region's pixels, so that the bound
+// follows the local contrast and flat content gives exactly equal D~.
+//
+// A lane walks down a window's columns with an 8-row register window of h and
+// keeps 8 keys (bits of D~, the low 6 bits replaced by the row), the 2
+// smallest of each of 4 sets of rows, and a bound of the others.  The best
+// matches cluster around a few positions (along a texture, in a few rows or
+// columns): lanes and row sets cut those clusters, so that the keys hold all
+// matches for all but a few blocks.
+//
+// Bound by VALU issue: 90 M wave instructions per 1080p frame (150 us of 195)
+// against bm3d_match_rows' 144 M; 53 KB of LDS, 3 workgroups per CU.  Two
+// grid rows per run share staging and sums (44 region rows instead of 80).
+// bm_range 16, block_step 4, 1920x1080, this kernel against bm3d_match_rows
+// (first passes, one lane): noisy images 0.195 / 0.251 ms, letterboxed 0.205
+// / 0.323, without noise 0.248 / 0.277, texture along columns 0.247 / 0.247.
+// ---------------------------------------------------------------------------
+
+// |D~ - D| <= kEps (N + box) for the candidate, where N = sum_j |c_j|^2 +
+// 8 |c7|^2 bounds every |R_k|^2: with u = 2^-24, the centring costs 4u (N +
+// box), h 3u N + 3u box, box 7u box, |R_k|^2 16u N, the correction's 7 chains
+// of 8 and their sums 30u N + 45u box, the main chain 27u N + 36u box and the
+// FP32 distance itself 24u (N + box): below 2^7 u = 2^-17 of N + box.
+// sqrt(box) <= sqrt(|R_k|^2) + sqrt(D) turns that into 3 kEps N + 2 kEps D.
+// Keys hold D~ + 4 kEps N, which is never negative.  With T the 8th smallest
+// of these (or an upper bound of it), 8 candidates have D <= T (1 + 3 kEps),
+// so the 8 nearest have D~ + 4 kEps N up to T (1 + 6 kEps) + 7 kEps N, which
+// select_threshold rounds up.
+constexpr float kEps = 0x1p-17f;
+__device__ __forceinline__ uint32_t select_threshold(uint32_t tk, float n)
+{
+    const float t = __uint_as_float(tk);
+    return __float_as_uint(t + (t * 0x1p-13f + n * (8.0f * kEps)));
+}
+// runs with pixels whose squares' 8-column sum is not below this (huge or
+// non-finite ones) are searched exactly; below it nothing here overflows
+constexpr float kMaxNorm = 1e30f;
+
+constexpr int kMaxAgain = 8;     // columns walked again (more: flat or periodic content)
+constexpr int kBoxRows = 13;     // box rows of a column per thread
+
+
+// The reference's FP32 distance of the candidate at window position (row, k):
+// cb the reference block, col0 window position (0, 0) of the row-major region
+// of row stride ss
+template <int CM>
+__device__ __forceinline__ float dist_at(const float *cb, const float *w0, int ss, int row, int k)
+{
+    float v[8];
+    const float *sp0 = w0 + row * ss + k;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float *sp = sp0 + j;
+        const float *cp = cb + min(k + j, 7);
+        float sv[8], cc[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            sv[i] = sp[i * ss];
+            cc[i] = cp[i * ss];
+        }
+        v[j] = col_ssd<CM>(cc, sv);
+    }
+    return ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+}
+
+// Half of dist_at: the sum of columns 0..3 (half 0) or 4..7 (half 1), which
+// the reference's tree adds last, so that two lanes make one distance
+template <int CM>
+__device__ __forceinline__ float half_dist_at(const float *cb, const float *w0, int ss, int row, int k, int half)
+{
+    float v[4];
+    const float *sp0 = w0 + row * ss + k + half * 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float *sp = sp0 + j;
+        const float *cp = cb + min(k + half * 4 + j, 7);
+        float sv[8], cc[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            sv[i] = sp[i * ss];
+            cc[i] = cp[i * ss];
+        }
+        v[j] = col_ssd<CM>(cc, sv);
+    }
+    return (v[0] + v[1]) + (v[2] + v[3]);
+}
+
+// N of the comment above from the |c_j|^2
+__device__ __forceinline__ float norm_bound(const float *cn)
+{
+    return (((cn[0] + cn[1]) + (cn[2] + cn[3])) + ((cn[4] + cn[5]) + (cn[6] + cn[7]))) + cn[7] * 8.0f;
+}
+
+// ascending sort of a bitonic sequence of 4
+__device__ __forceinline__ void bitonic4(uint32_t (&h)[4])
+{
+    const uint32_t a = min(h[0], h[2]), c = max(h[0], h[2]);
+    const uint32_t b = min(h[1], h[3]), d = max(h[1], h[3]);
+    h[0] = min(a, b);
+    h[1] = max(a, b);
+    h[2] = min(c, d);
+    h[3] = max(c, d);
+}
+
+// One level of row_eighth: lanes hold ascending lists of 4; the two lists of
+// 8 of lane pairs that CTRL mirrors onto each other become, in both, the
+// ascending list of their 8 smallest.  side: 0 in even lanes, ~0 in odd ones
+// (median with it is a minimum or a maximum).
+template <int CTRL>
+__device__ __forceinline__ void merge_low8(uint32_t (&h)[4], uint32_t side)
+{
+    uint32_t l[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        l[i] = min(h[i], dpp_mov<CTRL>(h[3 - i]));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        h[i] = med3_u32(l[i], dpp_mov<0xB1>(l[i]), side);  // quad_perm [1,0,3,2]
+    }
+    bitonic4(h);
+}
+
+// The 8th smallest of the 64 values that the 16 lanes of a row hold in
+// ascending lists of 4 (every lane of the row gets it)
+__device__ __forceinline__ uint32_t row_eighth(uint32_t (&h)[4], int lane)
+{
+    const uint32_t side = (lane & 1) ? ~0u : 0u;
+    uint32_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        o[i] = dpp_mov<0xB1>(h[3 - i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        h[i] = med3_u32(h[i], o[i], side);
+    }
+    bitonic4(h);                 // pairs: 8 ascending
+    merge_low8<0x1B>(h, side);   // quad_perm [3,2,1,0]: of 4 lanes
+    merge_low8<0x141>(h, side);  // row_half_mirror: of 8 lanes
+    uint32_t m = 0u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        m = max(m, min(h[i], dpp_mov<0x140>(h[3 - i])));  // row_mirror: of the row
+    }
+    return max(m, dpp_mov<0xB1>(m));
+}
+
+// sum over the 16 lanes of each row, in every lane
+__device__ __forceinline__ int row_sum16(int v, int lane)
+{
+    v += int(dpp_xor<1>(uint32_t(v), lane));
+    v += int(dpp_xor<2>(uint32_t(v), lane));
+    v += int(dpp_xor<4>(uint32_t(v), lane));
+    v += int(dpp_xor<8>(uint32_t(v), lane));
+    return v;
+}
+
+// the same of floats
+__device__ __forceinline__ float row_sum16f(float v, int lane)
+{
+    v += __uint_as_float(dpp_xor<1>(__float_as_uint(v), lane));
+    v += __uint_as_float(dpp_xor<2>(__float_as_uint(v), lane));
+    v += __uint_as_float(dpp_xor<4>(__float_as_uint(v), lane));
+    v += __uint_as_float(dpp_xor<8>(__float_as_uint(v), lane));
+    return v;
+}
+
+// keys below mine among the 16 of the lane's row (its rank); odd: whether the
+// odd lanes hold any
+__device__ __forceinline__ int row_rank16(uint64_t key, bool odd)
+{
+    int r = 0;
+#define VSFEEL_ROT(N)                                                                                       \
+    r += ((uint64_t(dpp_mov<0x120 + N>(uint32_t(key >> 32))) << 32) | dpp_mov<0x120 + N>(uint32_t(key))) < key
+    VSFEEL_ROT(2);
+    VSFEEL_ROT(4);
+    VSFEEL_ROT(6);
+    VSFEEL_ROT(8);
+    VSFEEL_ROT(10);
+    VSFEEL_ROT(12);
+    VSFEEL_ROT(14);
+    if (odd) {
+        VSFEEL_ROT(1);
+        VSFEEL_ROT(3);
+        VSFEEL_ROT(5);
+        VSFEEL_ROT(7);
+        VSFEEL_ROT(9);
+        VSFEEL_ROT(11);
+        VSFEEL_ROT(13);
+        VSFEEL_ROT(15);
+    }
+#undef VSFEEL_ROT
+    return r;
+}
+
+// Merges one candidate per lane (kNoKey where there is none) into the list,
+// keeping its 8 smallest keys: by ranks in rows of 16 lanes, from 64
+// candidates to 32, 16 and the 8 that meet the list in one row
+__device__ __forceinline__ void merge_nearest(TopList &T, uint64_t key, uint32_t xy, int lane)
+{
+    auto move = [&](int to) {
+        const uint32_t hi = uint32_t(__builtin_amdgcn_ds_permute(to * 4, int(uint32_t(key >> 32))));
+        const uint32_t lo = uint32_t(__builtin_amdgcn_ds_permute(to * 4, int(uint32_t(key))));
+        xy = uint32_t(__builtin_amdgcn_ds_permute(to * 4, int(xy)));
+        key = (uint64_t(hi) << 32) | lo;
+    };
+    // (equal keys only where there is no candidate: those take what ranks are
+    // left, which the row's lanes before them number)
+    auto rank = [&]() {
+        const uint64_t none = __ballot(key == kNoKey);
+        const uint32_t row = uint32_t(none >> (lane & 48)) & 0xFFFFu;
+        return row_rank16(key, true) + (key == kNoKey ? __popc(row & ((1u << (lane & 15)) - 1u)) : 0);
+    };
+    const int row = lane >> 4;
+    int r = rank();
+    move(r < 8 ? row * 8 + r : 32 + row * 8 + r - 8);
+    key = lane < 32 ? key : kNoKey;
+    r = rank();
+    move(lane < 32 ? (r < 8 ? row * 8 + r : 16 + row * 8 + r - 8) : lane);
+    key = lane < 16 ? key : kNoKey;
+    r = rank();
+    // the 8 smallest in lanes 8..15, the list in lanes 0..7
+    move(lane < 16 ? (r < 8 ? 8 + r : r - 8) : lane);
+    if (lane < 8) {
+        key = T.key;
+        xy = T.xy;
+    }
+    r = row_rank16(key, true);
+    // (two placeholders or none may tie: lower lanes first)
+    const uint64_t ties = __ballot(lane < 16 && key >= kPlaceholderKey);
+    if (key >= kPlaceholderKey) {
+        key = kPlaceholderKey;
+        xy = 0u;
+        r = 16 - __popcll(ties) + __popcll(ties & ((uint64_t(1) << lane) - 1u));
+    }
+    move(lane < 16 ? r : lane);
+    if (lane < 8) {
+        T.key = key;
+        T.xy = xy;
+    }
+}
+
+// med3_u32 as one instruction, which the compiler does not always find
+__device__ __forceinline__ uint32_t med3_single(uint32_t a, uint32_t b, uint32_t c)
+{
+    uint32_t m;
+    asm("v_med3_u32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+    return m;
+}
+
+// What a lane keeps of its window column: of each 4th row the 3 smallest keys
+struct ColumnKeys {
+    uint32_t best[4][3];
+    __device__ __forceinline__ void reset()
+    {
+#pragma unroll
+        for (int i = 0; i < 12; ++i) {
+            best[i / 3][i % 3] = ~0u;
+        }
+    }
+    __device__ __forceinline__ void insert(float d, uint32_t row, int set)
+    {
+        const uint32_t key = (__float_as_uint(d) & ~63u) | row;
+        uint32_t(&e)[3] = best[set];
+        e[2] = med3_single(e[1], e[2], key);
+        e[1] = med3_single(e[0], e[1], key);
+        e[0] = min(e[0], key);
+    }
+    // the smallest two of rows 0, 1 (mod 4) ascending, those of rows 2, 3, and
+    // the smallest third one, which no other candidate of the column is below
+    __device__ __forceinline__ void store(uint4 *q, uint32_t *bound) const
+    {
+        uint32_t a[4] = {best[0][0], best[0][1], best[1][1], best[1][0]};
+        uint32_t b[4] = {best[2][0], best[2][1], best[3][1], best[3][0]};
+        bitonic4(a);
+        bitonic4(b);
+        q[0] = make_uint4(a[0], a[1], a[2], a[3]);
+        q[1] = make_uint4(b[0], b[1], b[2], b[3]);
+        *bound = min(min(best[0][2], best[1][2]), min(best[2][2], best[3][2]));
+    }
+};
+
+// Window column of a lane walked downwards.  hp, bp, kp: the column's h, box
+// and corr from window row 0 on
+__device__ __forceinline__ void walk_column(const float (&c)[8], const float *hp, const float *bp, const float *kp,
+                                            int rh, ColumnKeys &K)
+{
+    float hw[8];
+#pragma unroll
+    for (int i = 0; i < 7; ++i) {
+        hw[i] = hp[i];
+    }
+    // 8 rows at a time, the last time with rows past the window (what is read
+    // for them is never used)
+    for (int r0 = 0; r0 < rh; r0 += 8) {
+        float h8[8], in[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            h8[u] = hp[r0 + 7 + u];
+            in[u] = bp[r0 + u] + kp[r0 + u];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            hw[(u + 7) & 7] = h8[u];
+            float d = in[u];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                d = __builtin_fmaf(c[i], hw[(u + i) & 7], d);
+            }
+            d = r0 + u < rh ? d : __uint_as_float(~0u);
+            K.insert(d, uint32_t(r0 + u), u & 3);
+        }
+    }
+}
+
+// A lane of a whole window does not stay in one column: texture along columns
+// would crowd all matches into one lane's keys.  Lane k walks column k for a
+// third of the rows, then the column a third of the window further on, and so
+// on (N rows and columns).
+template <int N>
+struct Shear {
+    static constexpr int kSeg = (N + 2) / 3;
+    static __device__ __forceinline__ int column(int k, int row)
+    {
+        const int c = k + row / kSeg * kSeg;
+        return c < N ? c : c - N;
+    }
+};
+
+// Lane k's candidates of a window of N x N.  hp, bp, kp: h, box and corr of
+// the window's first column from window row 0 on, with their column strides
+// (corr: of the first 7 columns, the 8th for the others)
+template <int N>
+__device__ __forceinline__ void walk_lane(const float (&c)[8], int k, const float *hp, int hr, const float *bp, int br,
+                                          const float *kp, int kr, ColumnKeys &K)
+{
+    constexpr int L = Shear<N>::kSeg;
+#pragma unroll
+    for (int r0 = 0; r0 < N; r0 += L) {
+        const int col = Shear<N>::column(k, r0);
+        const float *h = hp + col * hr + r0, *b = bp + col * br + r0, *q = kp + min(col, 7) * kr + r0;
+        float hw[8];
+#pragma unroll
+        for (int i = 0; i < 7; ++i) {
+            hw[i] = h[i];
+        }
+#pragma unroll
+        for (int r = 0; r < L && r0 + r < N; ++r) {
+            hw[(r + 7) & 7] = h[r + 7];
+            float d = b[r] + q[r];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                d = __builtin_fmaf(c[i], hw[(r + i) & 7], d);
+            }
+            K.insert(d, uint32_t(r0 + r), (r0 + r) & 3);
+        }
+    }
+}
+
+// The same for two blocks 4 rows apart: block rows 4..7 of the upper one are
+// rows 0..3 of the lower one, at the same distance from their candidates'
+// rows, so that 4 products are shared, and so are h and box.  c: -2 c7 of
+// their 12 rows; hp, bp: from the upper window's row 0 on
+template <int N>
+__device__ __forceinline__ void walk_lane_pair(const float (&c)[12], int k, const float *hp, int hr, const float *bp,
+                                               int br, const float *kp0, const float *kp1, int kr, ColumnKeys &K0,
+                                               ColumnKeys &K1)
+{
+    constexpr int L = Shear<N>::kSeg;
+#pragma unroll
+    for (int r0 = 0; r0 < N; r0 += L) {
+        const int col = Shear<N>::column(k, r0), ck = min(col, 7) * kr + r0;
+        const float *h = hp + col * hr + r0, *b = bp + col * br + r0, *q0 = kp0 + ck, *q1 = kp1 + ck;
+        float hw[12], bw[5];
+#pragma unroll
+        for (int i = 0; i < 11; ++i) {
+            hw[i] = h[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            bw[i] = b[i];
+        }
+#pragma unroll
+        for (int r = 0; r < L && r0 + r < N; ++r) {
+            hw[(r + 11) % 12] = h[r + 11];
+            bw[(r + 4) % 5] = b[r + 4];
+            float mid = c[4] * hw[(r + 4) % 12];
+            float d0 = bw[r % 5] + q0[r], d1 = bw[(r + 4) % 5] + q1[r];
+#pragma unroll
+            for (int i = 5; i < 8; ++i) {
+                mid = __builtin_fmaf(c[i], hw[(r + i) % 12], mid);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                d0 = __builtin_fmaf(c[i], hw[(r + i) % 12], d0);
+                d1 = __builtin_fmaf(c[i + 8], hw[(r + i + 8) % 12], d1);
+            }
+            K0.insert(d0 + mid, uint32_t(r0 + r), (r0 + r) & 3);
+            K1.insert(d1 + mid, uint32_t(r0 + r), (r0 + r) & 3);
+        }
+    }
+}
+
+// the group (radius 0) or the spatial top-8 (radius > 0) of one block from
+// its 8 nearest, candidate `rank` held by this lane (rank >= 8: none); sub:
+// the lane in its row of 16, all of which call this together
+__device__ __forceinline__ void write_nearest(const MatchArgs &A, uint64_t key, uint32_t xy, int rank, int blk, int x,
+                                              int y, int lane, bool act)
+{
+    const uint32_t d = uint32_t(key >> 32);
+    if (A.spatial) {
+        if (act && rank < 8) {
+            A.spatial[(long long)blk * 8 + rank] = make_uint2(d, xy);
+        }
+        return;
+    }
+    // the reference block is always a member (src/bm3d.comp:639-663)
+    const uint32_t self_xy = uint32_t(x) | (uint32_t(y) << 16);
+    const uint64_t in = __ballot(rank < 8 && xy == self_xy);
+    const int absent = (uint32_t(in >> (lane & 48)) & 0xFFFFu) == 0u ? 1 : 0;
+    rank += absent;
+    if (act && rank < 8) {
+        A.groups[(long long)blk * 8 + rank] = pack_entry(xy & 0xFFFFu, xy >> 16, uint32_t(A.radius));
+        if (A.dists) {
+            A.dists[(long long)blk * 8 + rank] = __uint_as_float(d);
+        }
+    }
+    if (act && absent && (lane & 15) == 0) {
+        A.groups[(long long)blk * 8] = pack_entry(uint32_t(x), uint32_t(y), uint32_t(A.radius));
+        if (A.dists) {
+            A.dists[(long long)blk * 8] = -1.0f;
+        }
+    }
+}
+
+// the same from a list (its lanes 0..7)
+__device__ __forceinline__ void write_list(const MatchArgs &A, const TopList &T, int blk, int x, int y, int lane)
+{
+    if (A.spatial) {
+        if (lane < 8) {
+            A.spatial[(long long)blk * 8 + lane] = make_uint2(uint32_t(T.key >> 32), T.xy);
+        }
+        return;
+    }
+    GroupList G;
+    G.e = __uint_as_float(uint32_t(T.key >> 32));
+    G.xy = T.xy;
+    G.z = A.radius;
+    finish_group(A, G, blk, x, y, lane);
+}
+
+// R: bm_range, s: block_step, VBC: grid rows per run; for frames at least as
+// large as the run's region (cols_geometry)
+template <int CM, int R, int s, int VBC>
+__global__ __launch_bounds__(256, 3) void bm3d_match_cols(MatchArgs A)
+{
+    extern __shared__ __align__(16) float clds[];
+    constexpr ColsGeometry G = cols_geometry(R, s, VBC);
+    constexpr ColsLayout L = cols_layout(G);
+    constexpr int N = 2 * R + 1, NB = G.nb, SS = G.ss, HR = G.hr, BR = (G.rrows - 7) | 1, KR = N | 1;
+    // pixels row-major, sums column-major: a lane per column reads them down
+    // its column with the row in the instruction's offset; odd column strides
+    // put the lanes on different banks
+    float *const src = clds;              // [rrows][SS] pixels
+    float *const hreg = clds + L.h;       // [columns][HR]
+    float *const box = clds + L.box;      // [columns][BR]
+    float *const qreg = clds + L.qk;      // [columns][HR], until box is made
+    // corr of grid row v, [NB][8][KR], after that; its keys, [NB][N][2], in
+    // corr's place
+    auto corr_of = [&](int v) { return clds + (v == 0 ? L.qk : L.keys); };
+    auto keys_of = [&](int v) { return reinterpret_cast<uint4 *>(clds + (v == 0 ? L.qk : L.keys)); };
+    uint32_t *const bounds = reinterpret_cast<uint32_t *>(clds + L.bounds);  // [blocks][N]
+    uint16_t *const stage0 = reinterpret_cast<uint16_t *>(clds + L.stage);   // [blocks][64] row | k << 6
+    float *const coef = clds + L.coef;                                   // [blocks][8]: -2 c7
+    float *const cnorm = clds + L.norm;                                  // [blocks][8]: |c_j|^2
+    int *const over = reinterpret_cast<int *>(clds + L.over);            // [blocks] left to a wavefront (below)
+    int *const flags = over + NB * VBC;  // blocks below D~'s resolution, some pixel huge or not finite, not flat, ...
+
+    const int W = A.width, H = A.height, pitch = A.pitch;
+    const int run = xcd_block_id();
+    const int runs_x = (A.nx + NB - 1) / NB;
+    const int rowp = run / runs_x;
+    const int bx0 = (run - rowp * runs_x) * NB, by0 = rowp * VBC;
+    const int nb = min(NB, A.nx - bx0), nv = min(VBC, A.ny - by0);
+    const int y_first = min(by0 * s, H - 8), y_last = min((by0 + nv - 1) * s, H - 8);
+    const int x_first = min(bx0 * s, W - 8), x_last = min((bx0 + nb - 1) * s, W - 8);
+    const int rx0 = max(x_first - R, 0), ry0 = max(y_first - R, 0);
+    const int ncols = min(x_last + R, W - 8) + 8 - rx0, nrows = min(y_last + R, H - 8) + 8 - ry0;
+    const float *plane = A.plane[A.radius] + (long long)ry0 * pitch + rx0;
+    const int t = threadIdx.x, lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+
+    // the source region: a lane per column, a wavefront per row (every fourth
+    // row), each lane issuing its batch of row loads before storing any
+    for (int c0 = 0; c0 < ncols; c0 += 64) {
+        const int c = c0 + lane;
+        const bool cok = c < ncols;
+        for (int r0 = wave; r0 < nrows; r0 += 4 * kStageBatch) {
+            float v[kStageBatch];
+#pragma unroll
+            for (int u = 0; u < kStageBatch; ++u) {
+                const int r = r0 + 4 * u;
+                v[u] = (cok && r < nrows) ? plane[r * pitch + c] : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < kStageBatch; ++u) {
+                const int r = r0 + 4 * u;
+                if (cok && r < nrows) {
+                    src[r * SS + c] = v[u];
+                }
+            }
+        }
+    }
+    {
+        // the columns past it that groups of 8 sums reach (those of the last
+        // row reach past it, too)
+        if (t < 4) {
+            flags[t] = 0;
+        }
+        const int pad = SS - ncols;
+        const float inv = 1.0f / float(max(pad, 1));
+        for (int i = t; i < nrows * pad + 8; i += 256) {
+            const int r = pad > 0 ? div_small(i, inv) : nrows;
+            src[r < nrows ? r * SS + ncols + (i - r * pad) : nrows * SS + (i - nrows * pad)] = 0.0f;
+        }
+    }
+    __syncthreads();
+
+    // the centre m: the mean of 8 pixels of the region (any finite value is
+    // valid; the mean of equal pixels is that pixel)
+    float m = 0.0f;
+    {
+        float e[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            e[i] = src[(((2 * i + 1) * nrows) >> 4) * SS + (((((i * 5) & 7) * 2 + 1) * ncols) >> 4)];
+        }
+        m = (((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]))) * 0.125f;
+        m = fabsf(m) < kMaxNorm ? m : 0.0f;
+    }
+
+    // Content without noise (bars, cartoons, clipped areas) matches far better
+    // than D~ resolves next to an edge.  A block's distance to itself one
+    // pixel to the right or below, from 16 of its pixels, stands for its
+    // nearest matches: a run where at least half of the blocks come below the
+    // resolution of D~ is searched exactly from the start
+    const int nblk = NB * nv;
+    for (int b0 = 0; b0 < nblk; b0 += 16) {
+        const int bl = b0 + (t >> 4), v = bl / NB, b = bl - v * NB;
+        const int xb = min((bx0 + min(b, nb - 1)) * s, W - 8), y = min((by0 + min(v, nv - 1)) * s, H - 8);
+        const float *cp = src + (y - ry0 + 2 * ((t >> 2) & 3)) * SS + (xb - rx0) + 2 * (t & 3);
+        const float c = cp[0], dx = cp[1] - c, dy = cp[SS] - c;
+        const float ex = row_sum16f(dx * dx, lane), ey = row_sum16f(dy * dy, lane);
+        const float e = (c - m) * (c - m), n = row_sum16f(e, lane);
+        // (4 times both for the block, twice N for the 16 columns of kEps' N)
+        if ((t & 15) == 0 && bl < nblk && b < nb && !(fminf(ex, ey) > n * (64.0f * kEps))) {
+            atomicAdd(flags, 1);
+        }
+    }
+    __syncthreads();
+    const bool exact = flags[0] * 2 >= nb * nv;
+
+    // the blocks' -2 c7 and |c_j|^2: a thread per block and column
+    for (int i = t; i < NB * nv * 8; i += 256) {
+        const int blk = i >> 3, j = i & 7;
+        const int v = blk / NB, b = blk - v * NB;
+        const int xb = min((bx0 + min(b, nb - 1)) * s, W - 8), y = min((by0 + v) * s, H - 8);
+        const float *cb = src + (y - ry0) * SS + (xb - rx0);
+        float n = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const float cj = cb[u * SS + j] - m;
+            n = __builtin_fmaf(cj, cj, n);
+        }
+        coef[i] = -2.0f * (cb[j * SS + 7] - m);
+        cnorm[i] = n;
+    }
+
+    // h and the 8-column sums of s^2 (q): 8 columns of a row per thread
+    uint32_t top_q = 0u;
+    if (!exact) {
+        const int items = (ncols >> 3) * nrows;  // (of ncols - 7 columns, rounded up)
+        const float inv = 1.0f / float(nrows);
+        for (int i = t; i < items; i += 256) {
+            const int ch = div_small(i, inv), r = i - ch * nrows, c = ch * 8;
+            const float4 *sp = reinterpret_cast<const float4 *>(src + r * SS + c);
+            float x[16], q[15];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float4 f = sp[k];
+                x[4 * k] = f.x - m;
+                x[4 * k + 1] = f.y - m;
+                x[4 * k + 2] = f.z - m;
+                x[4 * k + 3] = f.w - m;
+            }
+#pragma unroll
+            for (int k = 0; k < 14; ++k) {
+                q[k] = __builtin_fmaf(x[k], x[k], x[k + 1] * x[k + 1]);
+            }
+#pragma unroll
+            for (int k = 0; k < 12; ++k) {
+                q[k] = q[k] + q[k + 2];
+            }
+            float *const qo = qreg + c * HR + r, *const ho = hreg + c * HR + r;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const float e = q[k] + q[k + 4];
+                qo[k * HR] = e;
+                // (not negative: larger bits are larger values, infinity and NaN above all)
+                top_q = max(top_q, __float_as_uint(e));
+            }
+#pragma unroll
+            for (int k = 0; k < 14; ++k) {
+                x[k] = x[k] + x[k + 1];
+            }
+#pragma unroll
+            for (int k = 0; k < 12; ++k) {
+                x[k] = x[k] + x[k + 2];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                ho[k * HR] = x[k] + x[k + 4];
+            }
+        }
+    }
+    if (top_q >= __float_as_uint(kMaxNorm)) {
+        flags[1] = 1;
+    }
+    if (exact) {
+        // whether every pixel is m: all distances are 0 and scan order decides
+        bool same = true;
+        for (int r = wave; r < nrows; r += 4) {
+            for (int c = lane; c < ncols; c += 64) {
+                same = same && src[r * SS + c] == m;
+            }
+        }
+        if (!same) {
+            flags[2] = 1;
+        }
+    }
+    __syncthreads();
+    const bool wild = flags[1] != 0;
+    // (windows of fewer than 8 candidates in a row are searched)
+    const bool flat = exact && flags[2] == 0 && min(R, W - 8) + 1 >= 8;
+
+    // box: 8-row sums of q, kBoxRows rows of a column per thread
+    if (!exact) {
+        const int nbr = nrows - 7, nst = (nbr + kBoxRows - 1) / kBoxRows, nhc = ncols - 7;
+        const float inv = 1.0f / float(nhc);
+        for (int i = t; i < nst * nhc; i += 256) {
+            const int st = div_small(i, inv), c = i - st * nhc;
+            const int r0 = st * kBoxRows;
+            float p[kBoxRows + 7];
+#pragma unroll
+            for (int k = 0; k < kBoxRows + 7; ++k) {
+                p[k] = qreg[c * HR + r0 + k];  // (rows past the region are not used)
+            }
+#pragma unroll
+            for (int k = 0; k < kBoxRows + 6; ++k) {
+                p[k] = p[k] + p[k + 1];
+            }
+#pragma unroll
+            for (int k = 0; k < kBoxRows + 4; ++k) {
+                p[k] = p[k] + p[k + 2];
+            }
+#pragma unroll
+            for (int k = 0; k < kBoxRows; ++k) {
+                if (r0 + k < nbr) {
+                    box[c * BR + r0 + k] = p[k] + p[k + 4];
+                }
+            }
+        }
+    }
+    __syncthreads();
+
+    // corr, with |R_k|^2 = 8 |c_7|^2 + sum_{j = k..6} (|c_j|^2 - |c_7|^2) and
+    // the keys' offset: first the term of each column j = 0..6, a thread per
+    // block and column (j = 7: the constant of all later candidates), the
+    // rows split over the workgroup.  Two grid rows 4 rows apart with whole
+    // windows share terms (walk_column_pair)
+    constexpr bool kPairs = s == 4 && VBC == 2;
+    const bool pair = kPairs && nv == 2 && y_last == y_first + 4 && y_first >= R && y_last + R <= H - 8;
+    if (!exact) {
+        constexpr int per = NB * 8, nseg = 256 / per;
+        const int seg = t / per, i = t - seg * per;
+        const int b = i >> 3, j = i & 7;
+        const int xb = min((bx0 + min(b, nb - 1)) * s, W - 8), left = max(xb - R, 0);
+        auto base_of = [&](int v) {
+            const float *cn = cnorm + v * per + b * 8;
+            const float n7 = cn[7];
+            return j < 7 ? cn[j] - n7 : 8.0f * n7 + norm_bound(cn) * (4.0f * kEps);
+        };
+        // (of the centred columns, whose rounding the bound counts)
+        auto coef_of = [&](const float *cb) { return -2.0f * ((cb[j] - m) - (cb[7] - m)); };
+        if (kPairs && pair && seg < nseg) {
+            constexpr int kRows = (N + 256 / (NB * 8) - 1) / (256 / (NB * 8));
+            const float base0 = base_of(0), base1 = base_of(1);
+            const float *cb = src + (y_first - ry0) * SS + (xb - rx0);
+            float d[12], x[kRows + 11];
+#pragma unroll
+            for (int u = 0; u < 12; ++u) {
+                d[u] = coef_of(cb + u * SS);
+            }
+            const int r0 = seg * kRows;
+            const float *sp = src + r0 * SS + (left - rx0) + j;
+            // (rows past the region are read but not used)
+#pragma unroll
+            for (int u = 0; u < kRows + 11; ++u) {
+                x[u] = sp[u * SS] - m;
+            }
+            float *o0 = corr_of(0) + i * KR + r0, *o1 = corr_of(1) + i * KR + r0;
+#pragma unroll
+            for (int q = 0; q < kRows; ++q) {
+                float mid = d[4] * x[q + 4], e0 = base0, e1 = base1;
+#pragma unroll
+                for (int u = 5; u < 8; ++u) {
+                    mid = __builtin_fmaf(d[u], x[q + u], mid);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    e0 = __builtin_fmaf(d[u], x[q + u], e0);
+                    e1 = __builtin_fmaf(d[u + 8], x[q + u + 8], e1);
+                }
+                if (r0 + q < N) {
+                    o0[q] = j < 7 ? e0 + mid : base0;
+                    o1[q] = j < 7 ? e1 + mid : base1;
+                }
+            }
+        }
+        for (int v = 0; v < nv && !pair; ++v) {
+            const int y = min((by0 + v) * s, H - 8);
+            const int top = max(y - R, 0), rh = min(y + R, H - 8) - top + 1;
+            constexpr int kRows = 8;
+            const int len = (rh + nseg - 1) / nseg;
+            if (seg < nseg) {
+                const float base = base_of(v);
+                float d[8];
+                const float *cb = src + (y - ry0) * SS + (xb - rx0);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    d[u] = coef_of(cb + u * SS);
+                }
+                const float *sp = src + (top - ry0) * SS + (left - rx0) + j;
+                float *out = corr_of(v) + i * KR;
+                const int r1 = min((seg + 1) * len, rh);
+                for (int r = seg * len; r < r1; r += kRows) {
+                    float x[kRows + 7];
+#pragma unroll
+                    for (int u = 0; u < kRows + 7; ++u) {
+                        x[u] = sp[(r + u) * SS] - m;
+                    }
+#pragma unroll
+                    for (int q = 0; q < kRows; ++q) {
+                        float e = base;
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) {
+                            e = __builtin_fmaf(d[u], x[q + u], e);
+                        }
+                        if (r + q < r1) {
+                            out[r + q] = j < 7 ? e : base;
+                        }
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    // then their sums from each column on, a thread per block and row
+    for (int v = 0; v < nv && !exact; ++v) {
+        const int y = min((by0 + v) * s, H - 8);
+        const int rh = min(y + R, H - 8) - max(y - R, 0) + 1;
+        const float inv = 1.0f / float(rh);
+        for (int i = t; i < NB * rh; i += 256) {
+            const int b = div_small(i, inv), r = i - b * rh;
+            float *q = corr_of(v) + b * 8 * KR + r;
+            float e = q[7 * KR];
+#pragma unroll
+            for (int j = 6; j >= 0; --j) {
+                e += q[j * KR];
+                q[j * KR] = e;
+            }
+        }
+    }
+    __syncthreads();
+    // the windows' columns, a lane each
+    if (!exact) {
+        ColumnKeys K[VBC];
+#pragma unroll
+        for (int v = 0; v < VBC; ++v) {
+            K[v].reset();
+        }
+        const int b = t / N, k = t - b * N;
+        const int xb = min((bx0 + b) * s, W - 8);
+        const int left = max(xb - R, 0), rw = min(xb + R, W - 8) - left + 1;
+        if (b < nb && k < rw) {
+            if (kPairs && pair && rw == N) {
+                float c[12];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    c[u] = coef[b * 8 + u];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    c[u + 8] = coef[(NB + b) * 8 + u + 4];
+                }
+                walk_lane_pair<N>(c, k, hreg + (left - rx0) * HR, HR, box + (left - rx0) * BR, BR,
+                                  corr_of(0) + b * 8 * KR, corr_of(1) + b * 8 * KR, KR, K[0], K[VBC - 1]);
+            } else {
+#pragma unroll
+                for (int v = 0; v < VBC; ++v) {
+                    if (v < nv) {
+                        const int y = min((by0 + v) * s, H - 8);
+                        const int top = max(y - R, 0), rh = min(y + R, H - 8) - top + 1;
+                        float c[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) {
+                            c[u] = coef[(v * NB + b) * 8 + u];
+                        }
+                        const float *hp = hreg + (left - rx0) * HR + (top - ry0);
+                        const float *bp = box + (left - rx0) * BR + (top - ry0);
+                        const float *kp = corr_of(v) + b * 8 * KR;
+                        if (rw == N && rh == N) {
+                            walk_lane<N>(c, k, hp, HR, bp, BR, kp, KR, K[v]);
+                        } else {
+                            walk_column(c, hp + k * HR, bp + k * BR, kp + min(k, 7) * KR, rh, K[v]);
+                        }
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        if (t < NB * N) {
+#pragma unroll
+            for (int v = 0; v < VBC; ++v) {
+                K[v].store(keys_of(v) + t * 2, bounds + v * NB * N + t);
+            }
+        }
+    }
+    __syncthreads();
+
+    // the 8 nearest of each block, by a row of 16 lanes (4 blocks per
+    // wavefront at once)
+    const int sub = lane & 15;
+    for (int b0 = 0; b0 < nblk; b0 += 16) {
+        if (b0 + 4 * wave >= nblk) {
+            continue;  // whole wavefront
+        }
+        const int bi = b0 + 4 * wave + (lane >> 4);
+        const int bq = min(bi, nblk - 1);
+        const int v = bq / NB, b = min(bq - v * NB, nb - 1);
+        const int bl = v * NB + b;
+        const bool act = bi < nblk && bi == bl;
+        const int xb = min((bx0 + b) * s, W - 8), y = min((by0 + v) * s, H - 8);
+        const int left = max(xb - R, 0), top = max(y - R, 0);
+        const int rw = min(xb + R, W - 8) - left + 1, rh = min(y + R, H - 8) - top + 1;
+        if (exact) {
+            if (act && sub == 0) {
+                over[bl] = flat ? 0 : 65;
+            }
+            if (!flat) {
+                continue;
+            }
+            // the first 8 positions of the window's first row
+            write_nearest(A, uint64_t(0), uint32_t(left + sub) | (uint32_t(top) << 16), sub < 8 ? sub : 16,
+                          (by0 + v) * A.nx + bx0 + b, xb, y, lane, act);
+            continue;
+        }
+        const uint4 *kc = keys_of(v) + b * N * 2;
+        const float *cn = cnorm + bl * 8;
+        const uint32_t *bc = bounds + bl * N;
+        uint16_t *stage = stage0 + bl * 64;
+        const float n = norm_bound(cn);
+
+        // the 8th smallest of the columns' stored keys; a lane takes every
+        // 8th column's low or high 4 and keeps the 4 smallest
+        const int hf = sub & 1, c0 = sub >> 1;
+        uint32_t h[4] = {~0u, ~0u, ~0u, ~0u};
+        if (c0 < N) {
+            const uint4 q = kc[c0 * 2 + hf];
+            h[0] = q.x;
+            h[1] = q.y;
+            h[2] = q.z;
+            h[3] = q.w;
+        }
+        for (int c = c0 + 8; c < N; c += 8) {
+            const uint4 q = kc[c * 2 + hf];
+            h[0] = min(h[0], q.w);
+            h[1] = min(h[1], q.z);
+            h[2] = min(h[2], q.y);
+            h[3] = min(h[3], q.x);
+            bitonic4(h);
+        }
+        const uint32_t tk = row_eighth(h, lane) | 63u;
+        // (a candidate's D~ bits are at least its key's without the row)
+        const uint32_t lim = select_threshold(tk, n) | 63u;
+        // (fewer than 8 candidates: no 8th key)
+        const bool plain = act && !wild && tk < 0x7F000000u;
+
+        // the column of lane k's candidate in a window row
+        const bool whole = rw == N && rh == N;
+        auto column_of = [&](int k, int row) { return whole ? Shear<N>::column(k, row) : k; };
+        // the candidates at or below lim: positions to the stage (up to 64;
+        // the count may be more), but for lanes that may have seen more of
+        // them than their keys (again: bit q, lane q * 16 + sub)
+        int cnt = 0;
+        uint32_t again = 0;
+        if (plain) {
+            for (int c = c0; c < N; c += 8) {
+                const uint4 e = kc[c * 2 + hf];
+                const int have = (e.x <= lim) + (e.y <= lim) + (e.z <= lim) + (e.w <= lim);
+                cnt += bc[c] <= lim ? 0 : have;
+            }
+            for (int q = 0, c = sub; c < N; ++q, c += 16) {
+                again |= bc[c] <= lim ? 1u << q : 0u;
+            }
+        }
+        int staged = row_sum16(cnt, lane);
+        int pos = row_prefix_sum16(cnt) - cnt;
+        for (int c = c0; cnt != 0 && c < N; c += 8) {
+            const uint4 e = kc[c * 2 + hf];
+            auto put = [&](uint32_t key) {
+                const int r = int(key & 63u);
+                stage[pos++] = uint16_t(r | (column_of(c, r) << 6));
+            };
+            if (e.x <= lim && bc[c] > lim && pos < 64) {
+                put(e.x);
+                if (e.y <= lim && pos < 64) {
+                    put(e.y);
+                    if (e.z <= lim && pos < 64) {
+                        put(e.z);
+                        if (e.w <= lim && pos < 64) {
+                            put(e.w);
+                        }
+                    }
+                }
+            }
+        }
+        if (__ballot(again != 0) != 0) {
+            // their candidates once more, 16 rows at a time (flat or periodic
+            // content has many such lanes and is left to the exact search)
+            if (row_sum16(__popc(again), lane) > kMaxAgain) {
+                staged = 65;
+            }
+            const float *cf = coef + bl * 8;
+            const float *cb = src + (y - ry0) * SS + (xb - rx0);
+            const float *sp0 = src + (top - ry0) * SS + (left - rx0);
+            const float nr0 = 8.0f * cn[7] + n * (4.0f * kEps);
+            float c7[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                c7[u] = cf[u];
+            }
+            for (int q = 0; q * 16 < N; ++q) {
+                uint32_t seg = uint32_t(__ballot((again >> q) & 1u) >> (lane & 48)) & 0xFFFFu;
+                while (__ballot(seg != 0u && staged <= 64) != 0) {
+                    const bool on = seg != 0u && staged <= 64;
+                    const int k = on ? q * 16 + __ffs(seg) - 1 : 0;
+                    seg &= seg - 1u;
+                    for (int r0 = 0; r0 < rh; r0 += 16) {
+                        const int r = min(r0 + sub, rh - 1), c = min(column_of(k, r), rw - 1);
+                        const float *hp = hreg + (left - rx0 + c) * HR + (top - ry0);
+                        float d = box[(left - rx0 + c) * BR + (top - ry0) + r] + nr0;
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) {
+                            d = __builtin_fmaf(c7[u], hp[r + u], d);
+                        }
+                        if (__ballot(on && c < 7) != 0) {
+                            // the first columns' corr, which is gone by now
+                            float nr = 0.0f;
+                            for (int j = 6; __ballot(on && c <= j) != 0; --j) {
+                                float e = 0.0f;
+                                for (int u = 0; u < 8; ++u) {
+                                    e = __builtin_fmaf(-2.0f * ((cb[u * SS + j] - m) - (cb[u * SS + 7] - m)),
+                                                       sp0[(r + u) * SS + j] - m, e);
+                                }
+                                nr += c <= j ? e + (cn[j] - cn[7]) : 0.0f;
+                            }
+                            d += nr;
+                        }
+                        const bool in = on && r0 + sub < rh && __float_as_uint(d) <= lim;
+                        const uint32_t sm = uint32_t(__ballot(in) >> (lane & 48)) & 0xFFFFu;
+                        const int p = staged + __popc(sm & ((1u << sub) - 1u));
+                        if (in && p < 64) {
+                            stage[p] = uint16_t(r | (c << 6));
+                        }
+                        staged += __popc(sm);
+                    }
+                }
+            }
+        }
+        wave_lds_sync();
+        const float *cb = src + (y - ry0) * SS + (xb - rx0);
+        const float *w0 = src + (top - ry0) * SS + (left - rx0);
+        const bool few = plain && staged <= 16;
+        // their distances, two lanes each; even lanes then hold the first 8,
+        // odd ones the others (usually there are none)
+        const bool more = __ballot(few && staged > 8) != 0;
+        uint32_t e = few && c0 < staged ? stage[c0] : 0u;
+        float d = half_dist_at<CM>(cb, w0, SS, int(e & 63u), int(e >> 6), hf);
+        d = d + __uint_as_float(dpp_mov<0xB1>(__float_as_uint(d)));
+        bool valid = few && hf == 0 && c0 < staged;
+        if (more) {
+            const uint32_t e2 = few && 8 + c0 < staged ? stage[8 + c0] : 0u;
+            float d2 = half_dist_at<CM>(cb, w0, SS, int(e2 & 63u), int(e2 >> 6), hf);
+            d2 = d2 + __uint_as_float(dpp_mov<0xB1>(__float_as_uint(d2)));
+            if (hf == 1) {
+                e = e2;
+                d = d2;
+                valid = few && 8 + c0 < staged;
+            }
+        }
+        const int row = int(e & 63u), k = int(e >> 6);
+        valid = valid && __float_as_uint(d) < kFltMaxBits;
+        const uint64_t key = valid ? make_key(d, row * rw + k) : kNoKey;
+        // (lanes without a candidate tie at kNoKey, above every candidate)
+        const int rank = row_rank16(key, more);
+        const int nvalid = __popc(uint32_t(__ballot(valid) >> (lane & 48)) & 0xFFFFu);
+        const bool done = few && nvalid >= 8;
+        write_nearest(A, key, uint32_t(left + k) | (uint32_t(top + row) << 16), valid && done ? rank : 16,
+                      (by0 + v) * A.nx + bx0 + b, xb, y, lane, act && done);
+        if (act && sub == 0) {
+            over[bl] = done ? 0 : plain && staged > 16 && staged <= 64 ? staged : 65;
+        }
+    }
+    __syncthreads();
+
+    // the other blocks, a wavefront each: equal pixels (bars, clipped areas)
+    // with 8 distances of 0 in the window, or 17..64 staged candidates
+    for (int bl = wave; bl < nblk; bl += 4) {
+        const int v = bl / NB, b = bl - v * NB;
+        if (b >= nb || over[bl] == 0) {
+            continue;
+        }
+        int staged = over[bl];
+        const int xb = min((bx0 + b) * s, W - 8), y = min((by0 + v) * s, H - 8);
+        const int left = max(xb - R, 0), top = max(y - R, 0);
+        const int rw = min(xb + R, W - 8) - left + 1, rh = min(y + R, H - 8) - top + 1;
+        const float *cb = src + (y - ry0) * SS + (xb - rx0);
+        const float *w0 = src + (top - ry0) * SS + (left - rx0);
+        uint16_t *stage = stage0 + bl * 64;
+        TopList T;
+        list_reset(T);
+        const float c = cb[0];
+        if (rw <= 57 && __ballot(cb[(lane >> 3) * SS + (lane & 7)] == c) == ~uint64_t(0)) {
+            // the first 8 of distance 0 in scan order: the pixels of a row
+            // whose squared difference is 0 as a mask (a lane per column),
+            // the blocks of them by 8 columns and 8 rows of it
+            uint64_t rows[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                rows[i] = 0;
+            }
+            int have = 0;
+            const int col = min(lane, rw + 6);
+            for (int r0 = 0; r0 < rh + 7 && have < 8; r0 += 8) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int r = r0 + i;
+                    const float e = w0[min(r, rh + 6) * SS + col] - c;
+                    uint64_t z = __ballot(lane < rw + 7 && r < rh + 7 && e * e == 0.0f);
+                    z &= z >> 1;
+                    z &= z >> 2;
+                    z &= z >> 4;
+                    rows[i] = z;
+                    const uint64_t blocks = ((rows[0] & rows[1]) & (rows[2] & rows[3])) &
+                                            ((rows[4] & rows[5]) & (rows[6] & rows[7]));
+                    const int rank = have + int(__builtin_amdgcn_mbcnt_hi(
+                                                uint32_t(blocks >> 32),
+                                                __builtin_amdgcn_mbcnt_lo(uint32_t(blocks), 0)));
+                    if (r >= 7 && ((blocks >> lane) & 1u) && rank < 8) {
+                        stage[rank] = uint16_t((r - 7) | (lane << 6));
+                    }
+                    have += r >= 7 ? __popcll(blocks) : 0;
+                }
+            }
+            // (otherwise the stage is not what it was any more)
+            staged = have >= 8 ? 0 : 65;
+            wave_lds_sync();
+            if (have >= 8) {
+                const uint32_t e = stage[lane & 7];
+                T.key = 0u;
+                T.xy = uint32_t(left + int(e >> 6)) | (uint32_t(top + int(e & 63u)) << 16);
+            }
+        } else if (staged <= 64) {
+            const uint32_t e = lane < staged ? stage[lane] : 0u;
+            const int row = int(e & 63u), k = int(e >> 6);
+            const float d = dist_at<CM>(cb, w0, SS, row, k);
+            const uint64_t key =
+                lane < staged && __float_as_uint(d) < kFltMaxBits ? make_key(d, row * rw + k) : kNoKey;
+            merge_nearest(T, key, uint32_t(left + k) | (uint32_t(top + row) << 16), lane);
+        }
+        if (staged > 64) {
+            if (lane == 0) {
+                over[bl] = 65;
+                flags[3] = 1;
+            }
+            continue;
+        }
+        if (lane == 0) {
+            over[bl] = 0;
+        }
+        write_list(A, T, (by0 + v) * A.nx + bx0 + b, xb, y, lane);
+    }
+    __syncthreads();
+    if (flags[3] == 0) {
+        return;
+    }
+
+    // What is left (many near-equal distances, short windows, huge or
+    // non-finite pixels): the distances themselves, a window row per thread,
+    // as the sliding scan makes them (scan_row_sliding), from the source
+    // region once more, column-major; top-8 from the rows' keys (select16,
+    // select_wave).  xblk blocks of a grid row at a time.
+    const int CS = G.rrows | 1, DC = N, RHX = N;
+    uint32_t *const xstage = reinterpret_cast<uint32_t *>(clds + L.h);       // [4][64] staged positions
+    float *const region = reinterpret_cast<float *>(xstage + 256);           // [rcols][CS]
+    uint32_t *const rowtop = reinterpret_cast<uint32_t *>(region + G.rcols * CS);  // [xblk][RHX][3]
+    uint16_t *const dist = reinterpret_cast<uint16_t *>(rowtop + L.xblk * RHX * 3);  // [xblk][RHX][DC]
+    int *const list = reinterpret_cast<int *>(stage0);                       // [NB] blocks left, then their threshold
+    uint32_t *const xthr = reinterpret_cast<uint32_t *>(list + NB);
+    const uint32_t pm = pos_mask(DC);
+    for (int c0 = 0; c0 < ncols; c0 += 64) {
+        const int c = c0 + lane;
+        if (c < ncols) {
+            for (int r = wave; r < nrows; r += 4) {
+                region[c * CS + r] = src[r * SS + c];
+            }
+        }
+    }
+    for (int v = 0; v < nv; ++v) {
+        const int y = min((by0 + v) * s, H - 8);
+        const int top = max(y - R, 0), rh = min(y + R, H - 8) - top + 1;
+        __syncthreads();
+        int left_over = 0;
+        if (wave == 0) {
+            const bool in = lane < nb && over[v * NB + lane] != 0;
+            const uint64_t mask = __ballot(in);
+            if (in) {
+                list[__builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0)] = lane;
+            }
+            left_over = __popcll(mask);
+            if (lane == 0) {
+                flags[0] = left_over;
+            }
+        }
+        __syncthreads();
+        left_over = flags[0];
+        for (int q0 = 0; q0 < left_over; q0 += L.xblk) {
+            const int nq = min(L.xblk, left_over - q0);
+            for (int i = t; i < nq * rh; i += 256) {
+                const int q = div_small(i, 1.0f / float(rh)), r = i - q * rh;
+                const int xb = min((bx0 + list[q0 + q]) * s, W - 8);
+                const int left = max(xb - R, 0), right = min(xb + R, W - 8);
+                const float *cb = region + (xb - rx0) * CS + (y - ry0);
+                const uint3 t3 =
+                    scan_row_sliding<CM, 11>(cb, CS, region + (left - rx0) * CS + (top - ry0) + r, CS,
+                                             right - left + 1, dist + (q * RHX + r) * DC, pm);
+                uint32_t *o = rowtop + (q * RHX + r) * 3;
+                o[0] = t3.x;
+                o[1] = t3.y;
+                o[2] = t3.z;
+            }
+            __syncthreads();
+            for (int b0 = 4 * wave; b0 < nq; b0 += 16) {
+                const int q = b0 + (lane >> 4);
+                const bool act = q < nq;
+                const int qs = act ? q : 0;
+                const int bx = bx0 + list[q0 + qs], xb = min(bx * s, W - 8);
+                const int left = max(xb - R, 0), right = min(xb + R, W - 8);
+                const SpatialRows<CM> geo{right - left + 1, left, top, region + (xb - rx0) * CS + (y - ry0),
+                                          region + (left - rx0) * CS + (top - ry0), CS};
+                uint64_t key;
+                uint32_t kxy, thr;
+                const int staged = select16(rowtop + qs * RHX * 3, dist + qs * RHX * DC, DC, rh, geo, act, lane,
+                                            xstage + wave * 64 + (lane & 48), key, kxy, thr, pm);
+                if (act && staged <= 16) {
+                    if (A.spatial) {
+                        if (sub < 8) {
+                            A.spatial[(long long)((by0 + v) * A.nx + bx) * 8 + sub] =
+                                make_uint2(uint32_t(key >> 32), kxy);
+                        }
+                    } else {
+                        finish_group16(A, __uint_as_float(uint32_t(key >> 32)), kxy, (by0 + v) * A.nx + bx, xb, y,
+                                       sub);
+                    }
+                }
+                if (act && sub == 0) {
+                    xthr[q] = staged > 16 ? thr : ~0u;
+                    over[v * NB + list[q0 + q]] = staged > 16 ? 1 : 0;
+                }
+            }
+            __syncthreads();
+            for (int q = wave; q < nq; q += 4) {
+                if (over[v * NB + list[q0 + q]] == 0) {
+                    continue;
+                }
+                const int bx = bx0 + list[q0 + q], xb = min(bx * s, W - 8);
+                const int left = max(xb - R, 0), right = min(xb + R, W - 8);
+                const SpatialRows<CM> geo{right - left + 1, left, top, region + (xb - rx0) * CS + (y - ry0),
+                                          region + (left - rx0) * CS + (top - ry0), CS};
+                TopList T;
+                select_wave(rowtop + q * RHX * 3, dist + q * RHX * DC, DC, rh, geo, xthr[q], pm, lane,
+                            xstage + wave * 64, T);
+                write_list(A, T, (by0 + v) * A.nx + bx, xb, y, lane);
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Temporal predictive search after bm3d_match_rows (src/bm3d.comp:540-637),
 // one wavefront per ref block and both directions at once: half 0 (lanes
 // 0..31) follows frames r-1, r-2, .., half 1 frames r+1, r+2, ...  Each step
@@ -829,7 +2060,7 @@ __global__ __launch_bounds__(64) void bm3d_match_predictive(MatchArgs A)
 
     cur[lane] = A.plane[r][(long long)(y + (lane & 7)) * pitch + x + (lane >> 3)];
 
-    // the spatial top-8 (bm3d_match_rows) starts the group and predicts
+    // the spatial top-8 (bm3d_match_cols) starts the group and predicts
     TopList L;
     list_reset(L);
     {
@@ -1095,7 +2326,7 @@ __global__ __launch_bounds__(256) void bm3d_match(MatchArgs A)
     TopList L;
     list_reset(L);
     if (A.spatial) {
-        // done by bm3d_match_rows
+        // done by bm3d_match_cols
         const uint2 e = A.spatial[(long long)blk * 8 + (lane & 7)];
         if (lane < 8) {
             L.key = uint64_t(e.x) << 32;
@@ -2093,14 +3324,32 @@ hipError_t launch_match(const MatchArgs &a, int fp_mode, hipStream_t s, bool tem
         if (a.radius == 0) {
             rows.spatial = nullptr;
         }
+        // bm_range 16 at block_step 4 (the benchmark harness) takes the
+        // expanded distances, whose sums and selection cost the same for any
+        // window: worth it from about 1000 candidates on.  With run-time
+        // geometry they were slower (778x751, bm_range 12 at block_step 8:
+        // 43 us against 24), compiled for bm_range 9 not faster (640x360 at
+        // block_step 8: 18 against 17 us; 512x512 at 4: 23 against 27 us)
+        if (a.cols_vb > 0) {
+            auto cols = [&](auto kernel, int vb) {
+                const ColsGeometry g = cols_geometry(16, 4, vb);
+                const size_t clds = size_t(cols_layout(g).total) * sizeof(float);
+                const dim3 cgrid(((a.ny + vb - 1) / vb) * ((a.nx + g.nb - 1) / g.nb));
+                hipLaunchKernelGGL(kernel, cgrid, block, clds, s, rows);
+                return hipGetLastError();
+            };
+            if (a.cols_vb == 2) {
+                return fused ? cols(bm3d_match_cols<kFpAll, 16, 4, 2>, 2) : cols(bm3d_match_cols<kFpExplicit, 16, 4, 2>, 2);
+            }
+            return fused ? cols(bm3d_match_cols<kFpAll, 16, 4, 1>, 1) : cols(bm3d_match_cols<kFpExplicit, 16, 4, 1>, 1);
+        }
         const size_t lds = size_t(rows_lds_bytes(a.region_cols, a.region_rows, a.run_blocks, a.dist_cols));
         const dim3 rgrid(a.ny * a.runs_x);
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, rgrid, block, lds, s, rows);
             return hipGetLastError();
         };
-        // compiled run geometries: bm_range 16 at block_step 4 (the
-        // benchmark harness), bm_range 9 at block_step 8 (the plugin's
+        // compiled run geometries: bm_range 9 at block_step 8 (the plugin's
         // defaults) and at block_step 4 (the differentiable workload), where
         // the host derived exactly that geometry
         auto is = [&](int br, int st) {
@@ -2108,15 +3357,13 @@ hipError_t launch_match(const MatchArgs &a, int fp_mode, hipStream_t s, bool tem
             return a.bm_range == br && a.step == st && a.run_blocks == g.run_blocks &&
                    a.region_cols == g.region_cols && a.region_rows == g.region_rows && a.dist_cols == g.dist_cols;
         };
-        const int geo = is(16, 4) ? 1 : is(9, 8) ? 2 : is(9, 4) ? 3 : 0;
+        const int geo = is(9, 8) ? 2 : is(9, 4) ? 3 : 0;
         if (fused) {
-            return geo == 1   ? go(bm3d_match_rows<kFpAll, 16, 4>)
-                   : geo == 2 ? go(bm3d_match_rows<kFpAll, 9, 8>)
+            return geo == 2   ? go(bm3d_match_rows<kFpAll, 9, 8>)
                    : geo == 3 ? go(bm3d_match_rows<kFpAll, 9, 4>)
                               : go(bm3d_match_rows<kFpAll, 0, 0>);
         }
-        return geo == 1   ? go(bm3d_match_rows<kFpExplicit, 16, 4>)
-               : geo == 2 ? go(bm3d_match_rows<kFpExplicit, 9, 8>)
+        return geo == 2   ? go(bm3d_match_rows<kFpExplicit, 9, 8>)
                : geo == 3 ? go(bm3d_match_rows<kFpExplicit, 9, 4>)
                           : go(bm3d_match_rows<kFpExplicit, 0, 0>);
     }
