@@ -604,9 +604,10 @@ __device__ __forceinline__ bool survives(float d, uint32_t thr)
 // src/bm3d.comp:624-628).  Inserting entries one by one with ginsert8's
 // strict '<' leaves the 8 smallest of the group and the entries by
 // (distance, rank), where the group's members rank first in their order and
-// the entries after them in insertion order; so 8 entries at a time are
-// merged by one 16-lane sort of (distance bits, rank, z) keys: lanes 0..7
-// the group, lanes 8..15 the entries.  fkey[t - 1] / fxy[t - 1] hold step
+// the entries after them in insertion order.  So 8 entries at a time (lanes
+// 8..15, the group in lanes 0..7) every lane's place among the 16 is counted:
+// an entry's by two ballots, the group's (already sorted) by the entries
+// strictly below each member, 5 operations per entry (a 16-lane sort: 14).  fkey[t - 1] / fxy[t - 1] hold step
 // t's sorted (distance, seq) keys and positions of direction h in lanes
 // h * 32 + i (radius r <= 2).
 __device__ __forceinline__ void insert_steps(GroupList &G, const uint64_t (&fkey)[2], const uint32_t (&fxy)[2], int r,
@@ -624,21 +625,33 @@ __device__ __forceinline__ void insert_steps(GroupList &G, const uint64_t (&fkey
         const uint32_t e2 = uint32_t(__shfl(int(uint32_t(fkey[1] >> 32)), src));
         const uint32_t x1 = uint32_t(__shfl(int(fxy[0]), src));
         const uint32_t x2 = uint32_t(__shfl(int(fxy[1]), src));
-        uint64_t key = kNoKey;
-        uint32_t kxy = 0u;
+        uint32_t v = ~0u, vxy = 0u, vz = 0u;
         if (lane < 8) {
-            key = (uint64_t(__float_as_uint(G.e)) << 32) | (uint32_t(lane) << 8) | uint32_t(G.z);
-            kxy = G.xy;
+            v = __float_as_uint(G.e);
+            vxy = G.xy;
+            vz = uint32_t(G.z);
         } else if (entry) {
-            const uint32_t z = uint32_t(h ? r + t : r - t);
-            key = (uint64_t(t == 1 ? e1 : e2) << 32) | (uint32_t(lane) << 8) | z;
-            kxy = t == 1 ? x1 : x2;
+            v = t == 1 ? e1 : e2;
+            vxy = t == 1 ? x1 : x2;
+            vz = uint32_t(h ? r + t : r - t);
         }
-        sort16_dpp(key, kxy, lane);
+        int place = lane;
+        const int n = min(8, n_ins - c0);
+#pragma unroll 4
+        for (int j = 0; j < n; ++j) {
+            const uint32_t d = uint32_t(__builtin_amdgcn_readlane(int(v), 8 + j));
+            const uint32_t lt = uint32_t(__ballot(v < d)), le = uint32_t(__ballot(v <= d));
+            const int own = __popc((lt | (le & ((1u << (8 + j)) - 1u))) & 0xFFFFu);
+            place = lane == 8 + j ? own : place + (lane < 8 && d < v ? 1 : 0);
+        }
+        // (places 8..15, lanes 16.. and unused entries land past the group)
+        v = uint32_t(__builtin_amdgcn_ds_permute(place * 4, int(v)));
+        vxy = uint32_t(__builtin_amdgcn_ds_permute(place * 4, int(vxy)));
+        vz = uint32_t(__builtin_amdgcn_ds_permute(place * 4, int(vz)));
         if (lane < 8) {
-            G.e = __uint_as_float(uint32_t(key >> 32));
-            G.xy = kxy;
-            G.z = int(key & 0xFFu);
+            G.e = __uint_as_float(v);
+            G.xy = vxy;
+            G.z = int(vz);
         }
     }
 }
