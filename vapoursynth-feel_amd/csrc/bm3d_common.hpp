@@ -82,6 +82,13 @@ struct MatchArgs {
     // nonzero: the temporal search runs both directions in one wavefront
     // (bm3d_match_predictive; needs ps_num * (2 ps_range + 1) <= 32)
     int pred_pair;
+    // non-null: bm3d_match_steps makes the temporal search from the planes
+    // of pixels, 8-column and 8x8 sums there: of window position z, those of
+    // slot hb_slot[z], three planes of hb_plane elements at pitch hb_pitch
+    const float *hb;
+    int hb_pitch;
+    long long hb_plane;
+    int hb_slot[kMaxWindow];
     // precision form (operand != kOperandFp32): MFMA distances of the
     // spatial search from the reference frame's plane set (bm3d_planes,
     // layout below), runs of mfma_run_blocks ref blocks per workgroup
@@ -171,6 +178,12 @@ __host__ __device__ inline long long predictive_lds_bytes(int ps_num, int ps_ran
     const long long wh = 2LL * ps_range + 1;
     return 64LL * 8 + 64LL * 4 + 64LL * 4 + 4LL * 2 * ps_num * predictive_win_stride(ps_range) + 4LL * 64 * wh;
 }
+
+// planes of 8-column and 8x8 sums of one frame (bm3d_sum_planes): rows past
+// the frame that bm3d_match_steps may load (never used), and the largest
+// ps_range it takes (a window column per lane of 32)
+constexpr int kSumPlanePad = 40;
+constexpr int kStepsMaxRange = 15;
 
 // LDS bytes of bm3d_match_rows: survivor stages of its 4 wavefronts (64 keys
 // + positions each), per window row its 3 smallest distances and the

@@ -36,6 +36,8 @@ hipError_t launch_fill_zero(float *p, long long n, hipStream_t s);
 hipError_t launch_tile_reduce(const ReduceArgs &a, hipStream_t s);
 hipError_t launch_weight_box(const BoxArgs &a, hipStream_t s);
 hipError_t launch_gather(const GatherArgs &a, hipStream_t s);
+hipError_t launch_sum_planes(const float *src, int pitch, int width, int height, float *hb, int hb_pitch,
+                             long long hb_plane, hipStream_t s);
 hipError_t launch_planes(const float *src, int pitch, int width, int height, uint16_t *set, int operand,
                          hipStream_t s);
 hipError_t launch_tile_tables(int *tab, int width, int height, int tiles_x, int tiles_y, int tile_bx, int tile_by,
@@ -199,6 +201,15 @@ struct Instance {
     uint32_t *groups_l[kMaxLanes - 1] = {};
     float *scratch_l[kMaxLanes - 1] = {};
     uint16_t *psets_l[kMaxLanes - 1] = {};
+    // bm3d_match_steps: a lane's planes of sums (bm3d_sum_planes) of the
+    // 2 radius + 1 frames f whose numbers hb_frame holds, f in slot f mod
+    // (2 radius + 1).  A lane sums each frame itself: two lanes sum each twice
+    // (9 us a frame at 853x481), rather than ordering their streams by it.
+    // nullptr: bm3d_match without them (no use, or no room).
+    float *hb_l[kMaxLanes] = {};
+    int hb_frame[kMaxLanes][kMaxWindow];
+    int hb_pitch = 0;
+    long long hb_plane = 0;
     uint2 *spatial_l[kMaxLanes - 1] = {};
     float *origins_l[kMaxLanes - 1] = {};
     float *rec_l[kMaxLanes - 1] = {};
@@ -510,6 +521,9 @@ struct Instance {
         (void)hipFree(cell_count);
         (void)hipFree(cell_list);
         (void)hipFree(psets);
+        for (float *p : hb_l) {
+            (void)hipFree(p);
+        }
         for (int i = 0; i < kMaxLanes - 1; ++i) {
             (void)hipFree(groups_l[i]);
             (void)hipFree(scratch_l[i]);
@@ -579,6 +593,7 @@ struct Instance {
     float *res_slot(int slot) const { return res_buf + (long long)slot * tw * 2 * pe; }
     uint32_t *lane_groups() const { return lane ? groups_l[lane - 1] : groups; }
     float *lane_scratch() const { return lane ? scratch_l[lane - 1] : scratch; }
+    float *lane_hb() const { return hb_l[lane]; }
     uint16_t *lane_psets() const { return lane ? psets_l[lane - 1] : psets; }
     uint2 *lane_spatial() const { return lane ? spatial_l[lane - 1] : spatial; }
     float *lane_origins() const { return lane ? origins_l[lane - 1] : origins; }
@@ -618,6 +633,9 @@ struct Instance {
         m.cols_vb = cols_vb;
         m.t_rows = t_rows;
         m.pred_pair = pred_pair;
+        m.hb = lane_hb();
+        m.hb_pitch = hb_pitch;
+        m.hb_plane = hb_plane;
         m.operand = operand;
         if (operand != kOperandFp32) {
             m.pset = lane_psets();
@@ -629,11 +647,47 @@ struct Instance {
         return m;
     }
 
-    // block matching of one estimate: in the precision form first the plane
-    // set of the reference frame (the spatial search's operands), then the
-    // search
-    hipError_t match(const MatchArgs &m, const float *const *search, int in_pitch, hipStream_t s)
+    // forgets the frames whose sums the lanes hold: at the start and the end
+    // of everything but the host path, and after a failure there (what was
+    // enqueued may not have run)
+    void forget_sums()
     {
+        for (auto &l : hb_frame) {
+            std::fill(std::begin(l), std::end(l), -1);
+        }
+    }
+    struct SumsScope {
+        Instance &d;
+        bool keep = false;
+        ~SumsScope()
+        {
+            if (!keep) {
+                d.forget_sums();
+            }
+        }
+    };
+
+    // block matching of the estimate of frame n: in the precision form first
+    // the plane set of the reference frame (the spatial search's operands);
+    // for the temporal search the sums of the neighbour frames that the lane
+    // does not hold yet
+    hipError_t match(MatchArgs &m, int n, const float *const *search, int in_pitch, hipStream_t s)
+    {
+        for (int z = 0; z < tw && m.hb; ++z) {
+            const int f = clampi(n - radius + z, 0, nframes - 1), slot = f % tw;
+            m.hb_slot[z] = slot;
+            if (z == radius || hb_frame[lane][slot] == f) {
+                continue;
+            }
+            const hipError_t e = timed_launch(kKernelPlanes, s, [&] {
+                return launch_sum_planes(search[z], in_pitch, width, height, lane_hb() + 3 * slot * hb_plane, hb_pitch,
+                                         hb_plane, s);
+            });
+            if (e != hipSuccess) {
+                return e;
+            }
+            hb_frame[lane][slot] = f;
+        }
         if (operand != kOperandFp32) {
             const hipError_t e = timed_launch(kKernelPlanes, s, [&] {
                 return launch_planes(search[radius], in_pitch, width, height, lane_psets(), operand, s);
@@ -657,7 +711,7 @@ struct Instance {
     // fused_dst (radius 0, tiled, plain mode): the tile reduction writes the
     // aggregated frame there instead of the slice; fuses() says when it does
     bool fuses() const { return tiled && radius == 0; }
-    hipError_t estimate(const float *const *search, const float *const *input, int in_pitch,
+    hipError_t estimate(int n, const float *const *search, const float *const *input, int in_pitch,
                         float *stack, int stack_pitch, hipStream_t s, float *dists_out = nullptr,
                         int mode = kFilterPlain, const Saved &saved = Saved(), float *fused_dst = nullptr,
                         int fused_pitch = 0)
@@ -697,7 +751,7 @@ struct Instance {
         if (mode != kFilterApply) {
             MatchArgs m = match_args(search, in_pitch, dists_out);
             m.groups = table;
-            e = match(m, search, in_pitch, s);
+            e = match(m, n, search, in_pitch, s);
             if (e != hipSuccess) {
                 return e;
             }
@@ -1096,6 +1150,19 @@ std::string parse_args(const vsfeel_bm3d_args &a, Instance &d)
                 predictive_lds_bytes(d.ps_num, d.ps_range) <= 64 * 1024) {
                 d.pred_pair = 1;
             }
+            // larger window sets: bm3d_match_steps from about two wavefronts
+            // for every SIMD on (283x280, 4900 blocks, 2 windows of 17 rows:
+            // 35 us against the general search's 43; 341x230, 1218 blocks, 4
+            // of 15: 32 against 40, but 6 us more for the launch of the sums;
+            // 166x114, 408 blocks, 2 of 17: 36 against 28); a lane addresses
+            // all sums of its window's frames by 32-bit byte offsets
+            const int hp = (d.width + 15) & ~15;
+            const long long plane = (long long)hp * (d.height + kSumPlanePad);
+            if (d.radius <= 2 && !d.pred_pair && d.ps_range <= kStepsMaxRange && d.nref >= 8 * kComputeUnits &&
+                plane * 3 * d.tw * 4 < (1LL << 32)) {
+                d.hb_pitch = hp;
+                d.hb_plane = plane;
+            }
         }
     }
     if (d.operand != kOperandFp32) {
@@ -1240,6 +1307,16 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
         (e = hipMalloc(&d.dst_dev, plane)) != hipSuccess) {
         return dev_fail(e, "hipMalloc");
     }
+    // (without the room the search that needs none is taken)
+    auto alloc_sums = [&](int lane) {
+        if (d.hb_plane > 0 &&
+            hipMalloc(&d.hb_l[lane], size_t(d.hb_plane) * 3 * d.tw * sizeof(float)) != hipSuccess) {
+            d.hb_l[lane] = nullptr;
+            (void)hipGetLastError();
+        }
+    };
+    alloc_sums(0);
+    d.forget_sums();
     if (d.operand != kOperandFp32) {
         d.pset_bytes = (plane_set_bytes(d.width, d.height) + 255) & ~255LL;
         if ((e = hipMalloc(&d.psets, size_t(d.pset_bytes))) != hipSuccess) {
@@ -1368,6 +1445,7 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
                 }
             }
             for (int i = 0; i < d.lanes - 1; ++i) {
+                alloc_sums(i + 1);
                 if ((e = hipMalloc(&d.groups_l[i], size_t(d.nref) * 8 * sizeof(uint32_t))) != hipSuccess ||
                     (e = hipMalloc(&d.scratch_l[i], scratch_elems * sizeof(float))) != hipSuccess ||
                     (d.operand != kOperandFp32 &&
@@ -1551,6 +1629,9 @@ int vsfeel_bm3d_get_frame(vsfeel_bm3d *h, int32_t n, const float *const *clip_pl
             VSFEEL_HIP(hipStreamWaitEvent(cin, d.slot_ev[size_t(slot)], 0), "hipStreamWaitEvent");
         }
         d.src_frame[slot] = -1;  // until the upload is enqueued
+        for (int &held : d.hb_frame[0]) {
+            held = held == f ? -1 : held;
+        }
         // in the final pass the slot holds [ref][source] like the reference's ring
         for (int c = 0; c < d.clips; ++c) {
             VSFEEL_HIP(hipMemcpyAsync(d.src_slot(slot, c), o.stage[size_t(stage_of[i]) * d.clips + c],
@@ -1601,7 +1682,7 @@ int vsfeel_bm3d_get_frame(vsfeel_bm3d *h, int32_t n, const float *const *clip_pl
                 search[z] = d.src_slot(ring, 0);
                 input[z] = d.src_slot(ring, d.clips - 1);
             }
-            const hipError_t e = d.estimate(search, input, d.pitch, d.res_slot(slot_of[est_i[k]]), d.pitch, q,
+            const hipError_t e = d.estimate(m, search, input, d.pitch, d.res_slot(slot_of[est_i[k]]), d.pitch, q,
                                             nullptr, kFilterPlain, Instance::Saved(), o.dev, d.pitch);
             if (e != hipSuccess) {
                 return e;
@@ -1620,6 +1701,7 @@ int vsfeel_bm3d_get_frame(vsfeel_bm3d *h, int32_t n, const float *const *clip_pl
         VSFEEL_HIP(d.end_on(s), "hipEventRecord");
         return fail(err, err_len, VSFEEL_BM3D_EDEVICE, "launch for frame " + std::to_string(n) + " failed (test hook)");
     }
+    Instance::SumsScope sums{d};
     if (d.request_graphs && !d.timing) {
         // the kernels from the slot's graph for this recompute pattern: captured
         // on the idle capture stream, then updated into the slot's executable
@@ -1659,6 +1741,7 @@ int vsfeel_bm3d_get_frame(vsfeel_bm3d *h, int32_t n, const float *const *clip_pl
     } else {
         VSFEEL_HIP(enqueue(s), "launch");
     }
+    sums.keep = true;
     for (int k = 0; k < nest; ++k) {
         d.res_frame[size_t(slot_of[est_i[k]])] = r == 0 ? -1 : est_m[k];
     }
@@ -1765,6 +1848,9 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
             Instance &d;
             ~LaneReset() { d.lane = 0; }
         } lane_reset{d};
+        // (the caller may rewrite the clip between calls)
+        d.forget_sums();
+        Instance::SumsScope sums{d};
         std::vector<int> held(d.res_cap, -1);
         std::vector<int> slot_of(d.tw);
         std::vector<char> slot_read(d.res_cap, 0);  // slot_read[slot] recorded in this call
@@ -1801,7 +1887,7 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
                 const float *input[kMaxWindow];
                 device_window(d, clip, m, search, input);
                 // radius 0: the tile reduction writes the frame (fused aggregation)
-                e = d.estimate(search, input, clip->pitch, d.res_slot(slot), d.pitch, qs, nullptr, kFilterPlain,
+                e = d.estimate(m, search, input, clip->pitch, d.res_slot(slot), d.pitch, qs, nullptr, kFilterPlain,
                                Instance::Saved(), out + (int64_t)(n - first) * out_frame_stride, out_pitch);
                 if (e == hipSuccess && nlanes > 1 && !fused) {
                     e = hipEventRecord(d.lane_done[d.lane], qs);
@@ -1958,7 +2044,7 @@ int vsfeel_bm3d_process_device_static(const vsfeel_bm3d_args *args, const vsfeel
         device_window(d, clip, n, search, input);
         // radius 0: the tile reduction writes the frame (fused aggregation);
         // the frame's own slice is never touched, so no stack is passed
-        e = d.estimate(search, input, clip->pitch, nullptr, d.pitch, s, nullptr, kFilterPlain, Instance::Saved(),
+        e = d.estimate(n, search, input, clip->pitch, nullptr, d.pitch, s, nullptr, kFilterPlain, Instance::Saved(),
                        out + (int64_t)(n - first) * out_frame_stride, out_pitch);
     }
     d.tile_tables = nullptr;
@@ -2025,7 +2111,7 @@ int vsfeel_bm3d_forward_saved(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cli
         sv.masks = saved->masks + (int64_t)i * d.nref * 8;
         sv.weights = saved->weights + (int64_t)i * d.nref;
         if (e == hipSuccess) {
-            e = d.estimate(search, input, clip->pitch, d.res_slot(d.lane), d.pitch, qs, nullptr, kFilterSave, sv);
+            e = d.estimate(n, search, input, clip->pitch, d.res_slot(d.lane), d.pitch, qs, nullptr, kFilterSave, sv);
         }
         if (e == hipSuccess) {
             e = d.aggregate(n, slot_of, out + (int64_t)i * out_frame_stride, out_pitch, qs,
@@ -2082,7 +2168,7 @@ int vsfeel_bm3d_backward(vsfeel_bm3d *h, const float *grad_out, int32_t grad_pit
         sv.masks = saved->masks + (int64_t)i * d.nref * 8;
         sv.weights = saved->weights + (int64_t)i * d.nref;
         if (e == hipSuccess) {
-            e = d.estimate(y, y, d.pitch, d.res_slot(d.lane), d.pitch, qs, nullptr, kFilterApply, sv);
+            e = d.estimate(0, y, y, d.pitch, d.res_slot(d.lane), d.pitch, qs, nullptr, kFilterApply, sv);
         }
         if (e == hipSuccess) {
             e = d.aggregate(0, slot_of, grad_in + (int64_t)i * gin_frame_stride, gin_pitch, qs, nullptr, 0, true);
@@ -2119,8 +2205,10 @@ int vsfeel_bm3d_debug_groups(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *clip
     const float *search[kMaxWindow];
     const float *input[kMaxWindow];
     device_window(d, clip, m, search, input);
-    const MatchArgs a = d.match_args(search, clip->pitch, d.dists);
-    VSFEEL_HIP(d.match(a, search, clip->pitch, s), "match launch");
+    MatchArgs a = d.match_args(search, clip->pitch, d.dists);
+    d.forget_sums();
+    Instance::SumsScope sums{d};
+    VSFEEL_HIP(d.match(a, m, search, clip->pitch, s), "match launch");
     std::vector<uint32_t> packed(size_t(d.nref) * 8);
     VSFEEL_HIP(hipMemcpyAsync(packed.data(), d.groups, packed.size() * 4, hipMemcpyDeviceToHost, s), "hipMemcpy");
     if (dists) {
@@ -2163,7 +2251,9 @@ int vsfeel_bm3d_debug_estimate(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
     const float *search[kMaxWindow];
     const float *input[kMaxWindow];
     device_window(d, clip, m, search, input);
-    VSFEEL_HIP(d.estimate(search, input, clip->pitch, res, res_pitch, s), "estimate launch");
+    d.forget_sums();
+    Instance::SumsScope sums{d};
+    VSFEEL_HIP(d.estimate(m, search, input, clip->pitch, res, res_pitch, s), "estimate launch");
     VSFEEL_HIP(d.end_on(s), "hipEventRecord");
     VSFEEL_HIP(hipStreamSynchronize(s), "hipStreamSynchronize");
     return VSFEEL_BM3D_OK;

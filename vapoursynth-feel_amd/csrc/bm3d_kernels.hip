@@ -8,9 +8,11 @@
 //                         run, exact distances of a shortlist
 //   bm3d_match_predictive temporal predictive search after it (radius 1-2),
 //                         one wavefront per reference block, both directions
+//   bm3d_match_steps      the same for larger window sets, distances expanded
+//                         into sums of the frame (bm3d_sum_planes)
 //   bm3d_match            block matching one wavefront per reference block:
 //                         the exact metric (radius 3-4) and temporal searches
-//                         with window sets too wide for the kernel above
+//                         of small frames and wider windows
 //   bm3d_estimate(_tiled) 3-D DCT, hard threshold (or Wiener shrinkage),
 //                         inverse, weighted scatter into the estimate stack
 //   bm3d_tile_reduce      the tiles' accumulators into the frame's own slice
@@ -2288,6 +2290,564 @@ __global__ __launch_bounds__(64) void bm3d_match_predictive(MatchArgs A)
     finish_group(A, G, blk, x, y, lane);
 }
 
+// ---------------------------------------------------------------------------
+// Temporal predictive search of window sets too large for the kernel above
+// (ps_num windows of more than 32 rows together), one wavefront per ref block
+// and both directions at once, a half each.  Steps, keys and insertions are
+// those of that kernel; the distances are expanded as in bm3d_match_cols, but
+// in double, which this chip multiplies and adds as fast as single:
+//   D~ = |R_k|^2 + box - 2 sum_i c7[i] h(cx, cy + i) - 2 sum_{j = k..6} sum_i
+//        (c_j - c7)[i] s(left + j, cy + i)
+// from planes of s, h (8-column sums) and box (8x8 sums of squares) that
+// bm3d_sum_planes makes once per frame, of one pitch and behind one buffer
+// descriptor, so that the rows' offsets are scalar.  h and box are rounded to
+// single, for the L2s' sake (in double the windows of a grid row in flight did
+// not fit them: 20 M misses a launch against 1 M, 670 us against 480, at
+// 1920x1080, radius 2, 2 windows of 15 rows), so that D~ is the distance to
+// 2^-21 of N: the candidates that may be among the first ps_num are rarely
+// many more than ps_num; they get the reference's FP32 distance (column SSDs
+// and summation tree, 8 lanes each), which alone decides.  LW lanes (16 or 32)
+// take a window, a lane per column, and walk its rows with an 8-row register
+// window of h read straight from the planes: 16 operations per candidate, and
+// nothing staged but the 7 columns of the last term.  (The general search
+// puts the distances of a wavefront's windows into LDS, 42 operations each,
+// one window after the other: 853x481, block_step 5, radius 2, 3 windows of 11
+// rows, a frame with bars: 441 us, here 150; 1790x962, block_step 4, radius 2,
+// 4 windows of 17 rows: 2.90 ms, here 2.1.)  Bound by the three pipes it keeps
+// about evenly busy: VALU issue, LDS reads of corr's operands, L1 reads of h
+// and box.  Of window sets of up to 32 rows the kernel above is faster or as
+// fast (3 windows of 7 rows 244 us against 431, 2 of 9 rows 29 against 34; 2
+// of 15 rows 445 us against 398, but 30 us of sums).
+// ---------------------------------------------------------------------------
+// D~ is off by the roundings of h and box, 2^-24 (2 box + N) < 2^-21 (N + D)
+// with N = sum_j |c_j|^2 + 8 |c7|^2; keys hold D~ + kStepEps N (never
+// negative).  The FP32 distance is off by less than 2^-20 D and what its
+// squares lose below 2^-126.  (box is infinite, and D~ with it, where N or D
+// is: `huge` blocks evaluate every candidate.)
+constexpr float kStepEps = 0x1p-20f, kStepRel = 0x1p-17f, kStepTiny = 0x1p-119f;
+
+// LDS of one wavefront.  The strides spread a half wave's accesses over the
+// banks: rows (a lane per window row) as columns (one per lane, 8 of them).
+template <int LW>
+struct StepLds {
+    static constexpr int kWin = 64 / LW;       // windows at once
+    static constexpr int kRows = LW + 6;       // of a window's source
+    static constexpr int kWinStride = 8 * kRows;
+    double s[kWin * kWinStride];               // [window][7 columns][rows], then corr [window][8][rows]
+    double d[7 * 8];                           // -2 (c_j - c7)
+    double e[8];                               // |c_j|^2 - |c7|^2; e[7]: |c7|^2
+    double none[LW];                           // NaN: corr of no candidate
+    float cur[64];                             // [column][row]
+    uint32_t pos[64];                          // staged: row | k << 5 | window << 10
+    unsigned long long key[32];
+    uint32_t xy[32];
+};
+
+// what a wavefront's searches of one frame of each direction share; its
+// methods are called by all lanes
+template <int CM, int LW>
+struct StepSearch {
+    // keys: the row in the low bits, the pass above it
+    static constexpr int kRowBits = LW == 16 ? 4 : 5;
+    static constexpr uint32_t kPosMask = LW == 16 ? 63u : 255u;
+    static constexpr int kRows = StepLds<LW>::kRows, kWinStride = StepLds<LW>::kWinStride;
+
+    StepLds<LW> &S;
+    const int W, H, PR, PN, wh, npass;
+    const uint32_t P, HP4;  // elements of a row, bytes of a plane
+    const __amdgpu_buffer_rsrc_t planes;
+    double c7[8];           // -2 c7 (wave-uniform)
+
+    // the lane's window column (and row, for corr), and its window of the
+    // half's pass
+    static __device__ __forceinline__ int column(int lane) { return lane & (LW - 1); }
+    static __device__ __forceinline__ int sub_window(int lane) { return LW == 16 ? (lane >> 4) & 1 : 0; }
+
+    __device__ __forceinline__ StepSearch(const MatchArgs &A, StepLds<LW> &lds, int lane)
+        : S(lds), W(A.width), H(A.height), PR(A.ps_range), PN(A.ps_num), wh(2 * PR + 1), npass(LW == 16 ? (PN + 1) >> 1 : PN), P(uint32_t(A.hb_pitch)),
+          HP4(uint32_t(A.hb_plane) * 4u),
+          planes(__builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A.hb), 0,
+                                                   uint32_t(3 * (2 * A.radius + 1)) * HP4, 0x00020000))
+    {
+        const uint64_t b = __builtin_bit_cast(uint64_t, -2.0 * double(S.cur[56 + (lane & 7)]));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            c7[i] = __builtin_bit_cast(double, readlane_u64(b, i));
+        }
+    }
+
+    __device__ __forceinline__ float load(uint32_t at, uint32_t uniform) const
+    {
+        return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(planes, int(at), int(uniform), 0));
+    }
+
+    // D~ of the pass's windows around the predictors `pred` in the half's
+    // frame at byte offset `frame`: f(row, D~, inside) for each row of the
+    // lane's column (NaN where not inside the window)
+    template <class F>
+    __device__ __forceinline__ void walk(uint32_t pred, uint32_t frame, double base, int pass, int lane,
+                                         F f) const
+    {
+        const int half = lane >> 5, k = column(lane), win = lane / LW;
+        const int w = LW == 16 ? 2 * pass + sub_window(lane) : pass;
+        const uint32_t q = uint32_t(__shfl(int(pred), half * 32 + min(w, PN - 1)));
+        const int cx = int(q & 0xFFFFu), cy = int(q >> 16);
+        const int left = max(cx - PR, 0), top = max(cy - PR, 0);
+        const int rw = min(cx + PR, W - 8) - left + 1, rh = min(cy + PR, H - 8) - top + 1;
+        // (an empty asm keeps the rows' offsets from being computed before
+        // the steps, for more scalar registers than there are)
+        uint32_t P4 = P * 4u;
+        asm volatile("" : "+s"(P4));
+        const uint32_t at = frame + (uint32_t(top) * P + uint32_t(left)) * 4u;
+        const uint32_t col = at + uint32_t(min(k, rw - 1)) * 4u;
+        auto h_at = [&](int row) { return load(col, HP4 + uint32_t(row) * P4); };
+        auto b_at = [&](int row) { return load(col, 2u * HP4 + uint32_t(row) * P4); };
+        // the first 7 source columns: 8 lanes a row, a column each (the 8th
+        // lane's, and rows past the window, are not used)
+        {
+            constexpr int kRowsAt = LW / 8, kLoads = (kRows + kRowsAt - 1) / kRowsAt;
+            const int c = lane & 7, r0 = (lane & (LW - 1)) >> 3;
+            const uint32_t own = at + (uint32_t(r0) * P + uint32_t(min(c, 6))) * 4u;
+            double *out = S.s + win * kWinStride + c * kRows + r0;
+            float v[kLoads];
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) {
+                v[i] = load(own, uint32_t(i * kRowsAt) * P4);
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) {
+                if ((i + 1) * kRowsAt <= kRows || i * kRowsAt + r0 < kRows) {
+                    out[i * kRowsAt] = double(v[i]);
+                }
+            }
+        }
+        float h0[7];
+#pragma unroll
+        for (int i = 0; i < 7; ++i) {
+            h0[i] = h_at(i);
+        }
+        wave_lds_sync();
+        // corr, a lane per window row (k): from the last of the 7 columns to
+        // the first, then in their place (NaN for rows past the window)
+        {
+            double e[8];
+            e[7] = k < rh ? base : __builtin_nan("");
+            const double *sp = S.s + win * kWinStride + min(k, wh - 1);
+#pragma unroll
+            for (int j = 6; j >= 0; --j) {
+                double v = S.e[j];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    v = __builtin_fma(S.d[j * 8 + i], sp[j * kRows + i], v);
+                }
+                e[j] = e[j + 1] + v;
+                if (j & 1) {
+                    __builtin_amdgcn_sched_barrier(0);  // two columns' operands at once
+                }
+            }
+            wave_lds_sync();
+            double *out = S.s + win * kWinStride + k;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                out[j * kRows] = e[j];
+            }
+        }
+        wave_lds_sync();
+        const bool inside = w < PN && k < rw;
+        const double *kp = inside ? S.s + win * kWinStride + min(k, 7) * kRows : S.none;
+        double hw[8];
+#pragma unroll
+        for (int i = 0; i < 7; ++i) {
+            hw[i] = double(h0[i]);
+        }
+        constexpr int kBatch = 8;
+#pragma unroll 1
+        for (int r0 = 0; r0 < wh; r0 += kBatch) {
+            float h8[kBatch], b8[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                h8[u] = h_at(r0 + u + 7);
+                b8[u] = b_at(r0 + u);
+            }
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                hw[(u + 7) & 7] = double(h8[u]);
+                double d = double(b8[u]) + kp[r0 + u];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    d = __builtin_fma(c7[i], hw[(u + i) & 7], d);
+                }
+                f(r0 + u, float(d), inside && r0 + u < rh);
+            }
+        }
+    }
+
+    // (distance, seq) key and position of staged candidate p of half h, whose
+    // frame lies at byte offset `frame`, by the 8 lanes of a group (a column
+    // each; valid in the group's first lane)
+    __device__ __forceinline__ void evaluate(uint32_t pred, uint32_t frame, uint32_t p, int h, bool valid,
+                                             int lane, uint64_t &key, uint32_t &xy) const
+    {
+        const int row = int(p & 31u), kc = int((p >> 5) & 31u), w = int(p >> 10), j = lane & 7;
+        const uint32_t q = uint32_t(__shfl(int(pred), h * 32 + w));
+        const int cx = int(q & 0xFFFFu), cy = int(q >> 16);
+        const int left = max(cx - PR, 0), top = max(cy - PR, 0), rw = min(cx + PR, W - 8) - left + 1;
+        const int px = valid ? left + kc : 0, py = valid ? top + row : 0;
+        const uint32_t at = frame + (uint32_t(py) * P + uint32_t(px + j)) * 4u;
+        const int a = min(kc + j, 7) * 8;
+        float cc[8], sv[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            cc[i] = S.cur[a + i];
+            sv[i] = load(at, uint32_t(i) * P * 4u);
+        }
+        float v = col_ssd<CM>(cc, sv);
+        v = v + __uint_as_float(dpp_mov<0x101>(__float_as_uint(v)));
+        v = v + __uint_as_float(dpp_mov<0x102>(__float_as_uint(v)));
+        v = v + __uint_as_float(dpp_mov<0x104>(__float_as_uint(v)));
+        key = valid && __float_as_uint(v) < kFltMaxBits ? make_key(v, w * wh * wh + row * rw + kc) : kNoKey;
+        xy = uint32_t(px) | (uint32_t(py) << 16);
+    }
+};
+
+// The step's first ps_num keys of half h when more candidates than its stage
+// holds lie below `lim` (ties), or a lane may have seen more than it kept:
+// those of another walk in scan order, evaluated 8 at a time until ps_num
+// distances are 0.  The keys and positions return in lanes 0..ps_num-1.  Not
+// inlined: its registers would be taken from every step.
+struct StepKeys {
+    uint64_t key;
+    uint32_t xy;
+};
+template <int CM, int LW>
+__device__ __attribute__((noinline)) StepKeys steps_all(const __attribute__((address_space(4))) MatchArgs *args,
+                                                        __attribute__((address_space(3))) StepLds<LW> *lds, int h_,
+                                                        uint32_t frame, uint32_t lim, uint32_t pred, double base)
+{
+    const uint64_t ap = reinterpret_cast<uint64_t>(args);
+    const MatchArgs &A = *(const MatchArgs *)(const __attribute__((address_space(4))) MatchArgs *)(
+        (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(ap >> 32)))) << 32) |
+        uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(ap)))));
+    const int h = __builtin_amdgcn_readfirstlane(h_);
+    const int lane = lane_id();
+    StepLds<LW> &S = *(StepLds<LW> *)lds;
+    const StepSearch<CM, LW> T(A, S, lane);
+    TopList L;
+    list_reset(L);
+    const uint32_t at = uint32_t(__builtin_amdgcn_readlane(int(frame), h * 32));
+    bool ended = false;
+    int held = 0;
+    auto flush = [&]() {
+        wave_lds_sync();
+        for (int e0 = 0; e0 < held && !ended; e0 += 8) {
+            const int e = e0 + (lane >> 3);
+            uint64_t key;
+            uint32_t xy;
+            T.evaluate(pred, at, S.pos[e & 63], h, e < held, lane, key, xy);
+            key = (lane & 7) == 0 ? key : kNoKey;
+            if (__ballot(key < readlane_u64(L.key, T.PN - 1)) != 0) {
+                list_merge_rounds(L, key, xy, lane, T.PN);
+            }
+            ended = uint32_t(readlane_u64(L.key, T.PN - 1) >> 32) == 0u;
+        }
+        held = 0;
+        wave_lds_sync();
+    };
+    for (int pass = 0; pass < T.npass && !ended; ++pass) {
+        uint32_t rows = 0u;
+        T.walk(pred, frame, base, pass, lane, [&](int row, float d, bool inside) {
+            rows |= (lane >> 5) == h && inside && __float_as_uint(d) <= lim ? 1u << row : 0u;
+        });
+        const int w0 = LW == 16 ? 2 * pass : pass;
+        for (int ws = 0; ws < (LW == 16 ? 2 : 1) && !ended; ++ws) {
+            for (int row = 0; row < T.wh && !ended; ++row) {
+                const bool in = T.sub_window(lane) == ws && (rows >> row) & 1u;
+                const uint64_t mask = __ballot(in);
+                if (mask == 0) {
+                    continue;
+                }
+                const int c = __popcll(mask);
+                if (held >= 8) {
+                    flush();  // (at most 32 then fit)
+                }
+                if (in) {
+                    S.pos[held + int(__builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32),
+                                                               __builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0)))] =
+                        uint32_t(row) | (uint32_t(T.column(lane)) << 5) | (uint32_t(w0 + ws) << 10);
+                }
+                held += c;
+            }
+        }
+    }
+    if (!ended) {
+        flush();
+    }
+    return {L.key, L.xy};
+}
+
+template <int CM, int LW>
+__global__ __launch_bounds__(256, 4) void bm3d_match_steps(MatchArgs A)
+{
+    __shared__ StepLds<LW> lds_all[4];
+    const int lane = lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    const int blk = xcd_block_id() * 4 + wave;
+    if (blk >= A.nx * A.ny) {
+        return;  // whole wavefront; no workgroup barrier follows
+    }
+    StepLds<LW> &S = lds_all[wave];
+    const int by = blk / A.nx, bx = blk - by * A.nx, r = A.radius;
+    const int x = min(bx * A.step, A.width - 8), y = min(by * A.step, A.height - 8);
+
+    // the reference block, its coefficients and norms
+    S.cur[lane] = A.plane[r][(long long)(y + (lane & 7)) * A.pitch + x + (lane >> 3)];
+    wave_lds_sync();
+    const StepSearch<CM, LW> T(A, S, lane);
+    const int PN = T.PN;
+    constexpr int kRowBits = T.kRowBits;
+    constexpr uint32_t pm = T.kPosMask;
+    // the smallest keys a lane keeps (one more is the bound of the rest)
+    constexpr int NK = 4;
+    if (lane < 56) {
+        S.d[lane] = -2.0 * (double(S.cur[lane]) - double(S.cur[56 + (lane & 7)]));
+    }
+    double norm = 0.0;  // |c_j|^2 of column j = lane & 7
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const double c = double(S.cur[(lane & 7) * 8 + i]);
+        norm = __builtin_fma(c, c, norm);
+    }
+    const double norm7 = __builtin_bit_cast(double, readlane_u64(__builtin_bit_cast(uint64_t, norm), 7));
+    if (lane < 8) {
+        S.e[lane] = lane < 7 ? norm - norm7 : norm;
+    }
+    if (lane < LW) {
+        S.none[lane] = __builtin_nan("");
+    }
+    // N, rounded up
+    float v = float(norm);
+    v += __uint_as_float(dpp_xor<1>(__float_as_uint(v), lane));
+    v += __uint_as_float(dpp_xor<2>(__float_as_uint(v), lane));
+    v += __uint_as_float(dpp_xor<4>(__float_as_uint(v), lane));
+    const bool huge = v > 1e28f || norm7 > 1e27;
+    const float margin = (v + 8.0f * float(norm7)) * (1.0f + 0x1p-20f) * kStepEps + kStepTiny;
+    const double base = __builtin_fma(8.0, norm7, double(margin));
+    wave_lds_sync();
+
+    // the spatial top-8 starts the group and predicts
+    GroupList G;
+    uint32_t pred;
+    bool flat;
+    {
+        const uint2 e = A.spatial[(long long)blk * 8 + (lane & 7)];
+        flat = __builtin_amdgcn_readlane(int(e.x), 7) == 0;
+        G.e = lane < 8 ? __uint_as_float(e.x) : FLT_MAX;
+        G.xy = lane < 8 ? e.y : 0u;
+        G.z = r;
+        pred = e.y;  // lanes h*32 + i (i < 8): predictor i
+    }
+    uint64_t fkey[2] = {kNoKey, kNoKey};  // frame top of steps 1, 2 (lanes h*32 + i)
+    uint32_t fxy[2] = {0u, 0u};
+#pragma unroll 1
+    for (int t = 1; t <= r; ++t) {
+        // (an empty asm keeps what follows from the lane alone, above all its
+        // masks, from being computed before the steps and kept in scalar
+        // registers that the rows' offsets need)
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int half = ln >> 5, sl = ln & 31;
+        // byte offset of the half's frame in the planes
+        const uint32_t frame = uint32_t(half ? A.hb_slot[r + t] : A.hb_slot[r - t]) * (3u * T.HP4);
+        // a block with 8 equals in its own frame (bars, mattes) usually finds
+        // as many at the start of its first window: the first ps_num
+        // distances of 0 in scan order are the step's result
+        uint64_t key = kNoKey;
+        uint32_t kxy = 0u;
+        bool done = false;
+        if (flat) {
+            const int cx = __shfl(int(pred), half * 32) & 0xFFFF;
+            const int rw = min(cx + T.PR, A.width - 8) - max(cx - T.PR, 0) + 1;
+            for (int e0 = 0; e0 < 8; e0 += 4) {
+                const int e = e0 + (sl >> 3);
+                T.evaluate(pred, frame, uint32_t(e) << 5, half, e < rw, ln, key, kxy);
+                if ((ln & 7) == 0) {
+                    S.key[half * 16 + e] = key;
+                    S.xy[half * 16 + e] = kxy;
+                }
+            }
+            wave_lds_sync();
+            key = sl < 8 ? S.key[half * 16 + sl] : kNoKey;
+            kxy = sl < 8 ? S.xy[half * 16 + sl] : 0u;
+            wave_lds_sync();
+            sort16_dpp(key, kxy, ln);
+            done = __popcll(__ballot(sl == PN - 1 && (key >> 32) == 0)) == 2;
+        }
+        if (!done) {
+            uint32_t m[NK + 1];
+#pragma unroll
+            for (int i = 0; i <= NK; ++i) {
+                m[i] = ~0u;
+            }
+            for (int pass = 0; pass < T.npass; ++pass) {
+                T.walk(pred, frame, base, pass, ln, [&](int row, float d, bool) {
+                    const uint32_t key = (__float_as_uint(d) & ~pm) | uint32_t(pass << kRowBits) | uint32_t(row);
+#pragma unroll
+                    for (int i = NK; i > 0; --i) {
+                        m[i] = med3_u32(m[i - 1], m[i], key);
+                    }
+                    m[0] = min(m[0], key);
+                });
+            }
+
+            // the half's ps_num-th smallest key bounds the ps_num-th distance;
+            // candidates up to that and its margin are staged
+            uint32_t tk = ~0u;
+            {
+                uint32_t h[NK];
+#pragma unroll
+                for (int i = 0; i < NK; ++i) {
+                    h[i] = m[i];
+                }
+                int taken = 0;
+                for (int it = 0; it < PN; ++it) {
+                    const uint32_t mn = half_min32_u32(h[0], ln);
+                    const bool hit = h[0] == mn;
+                    if (taken < PN) {
+                        taken += __popc(uint32_t(__ballot(hit) >> (half * 32)));
+                        tk = mn;
+                    }
+                    if (hit) {
+#pragma unroll
+                        for (int i = 0; i + 1 < NK; ++i) {
+                            h[i] = h[i + 1];
+                        }
+                        h[NK - 1] = ~0u;
+                    }
+                }
+            }
+            // (fewer than ps_num distances below infinity: all of them)
+            const float tf = __uint_as_float(tk | pm);
+            const float lf = tf + (tf * kStepRel + margin);
+            const uint32_t lim = (tk | pm) < 0x7F800000u && lf < FLT_MAX ? (__float_as_uint(lf) | pm) : (0x7F800000u | pm);
+            int staged = 0;
+#pragma unroll
+            for (int i = 0; i < NK; ++i) {
+                const bool in = m[i] <= lim;
+                const uint64_t mask = __ballot(in);
+                const uint32_t lo = uint32_t(mask), hi = uint32_t(mask >> 32);
+                const int at = staged + int(half ? __builtin_amdgcn_mbcnt_hi(hi, 0u) : __builtin_amdgcn_mbcnt_lo(lo, 0u));
+                staged += half ? __popc(hi) : __popc(lo);
+                if (in && at < 16) {
+                    const uint32_t pass = (m[i] & pm) >> kRowBits, row = m[i] & ((1u << kRowBits) - 1u);
+                    const uint32_t w = LW == 16 ? 2 * pass + uint32_t(T.sub_window(ln)) : pass;
+                    S.pos[half * 32 + at] = row | (uint32_t(T.column(ln)) << 5) | (w << 10);
+                }
+            }
+            const uint64_t over = __ballot(huge || staged > 16 || m[NK] <= lim);
+            wave_lds_sync();
+            const int most = max(__builtin_amdgcn_readlane(staged, 0), __builtin_amdgcn_readlane(staged, 32));
+            for (int e0 = 0; e0 < min(most, 16); e0 += 4) {
+                const int e = e0 + (sl >> 3);
+                uint64_t key;
+                uint32_t xy;
+                T.evaluate(pred, frame, S.pos[half * 32 + e], half, e < staged, ln, key, xy);
+                if ((ln & 7) == 0) {
+                    S.key[half * 16 + e] = key;
+                    S.xy[half * 16 + e] = xy;
+                }
+            }
+            wave_lds_sync();
+            key = sl < 16 && sl < staged ? S.key[half * 16 + sl] : kNoKey;
+            kxy = sl < 16 && sl < staged ? S.xy[half * 16 + sl] : 0u;
+            wave_lds_sync();
+            if (most <= 4) {
+                sort16_step<2, 1>(key, kxy, ln);
+                sort16_step<4, 2>(key, kxy, ln);
+                sort16_step<4, 1>(key, kxy, ln);
+            } else {
+                sort16_dpp(key, kxy, ln);
+            }
+            if (!(key < kPlaceholderKey)) {
+                key = kPlaceholderKey;  // fewer than ps_num candidates in the step
+                kxy = 0u;
+            }
+            for (int h = 0; h < 2; ++h) {
+                if (uint32_t(over >> (h * 32)) != 0u) {
+                    const uint32_t all = huge ? ~0u : uint32_t(__builtin_amdgcn_readlane(int(lim), h * 32));
+                    const StepKeys f = steps_all<CM, LW>(
+                        (const __attribute__((address_space(4))) MatchArgs *)__builtin_amdgcn_kernarg_segment_ptr(),
+                        (__attribute__((address_space(3))) StepLds<LW> *)&S, h, frame, all, pred, base);
+                    const uint64_t fk = shfl64(f.key, sl & 7);
+                    const uint32_t fx = uint32_t(__shfl(int(f.xy), sl & 7));
+                    if (half == h && sl < 8) {
+                        key = fk;
+                        kxy = fx;
+                    }
+                }
+            }
+        }
+        if (t == 1) {
+            fkey[0] = key;
+            fxy[0] = kxy;
+        } else {
+            fkey[1] = key;
+            fxy[1] = kxy;
+        }
+        pred = kxy;
+    }
+    insert_steps(G, fkey, fxy, r, PN, lane);
+    finish_group(A, G, blk, x, y, lane);
+}
+
+// s, h and box of one frame for bm3d_match_steps, rounded from double: h(x, y) the sum of
+// the pixels at x .. x+7, box(x, y) that of the squares of the 8x8 block
+// there.  A workgroup makes a tile of 64 x 16; rows past the frame (whose
+// values no search uses) are left out.  Bound by its 12 bytes written per
+// pixel (853x481: 8 us with the launch; 3840x2160: 44 us, 2.7 TB/s).
+constexpr int kSumW = 64, kSumH = 16;
+__global__ __launch_bounds__(256) void bm3d_sum_planes(const float *src, int pitch, int width, int height, float *hb,
+                                                       long long hplane, int hpitch)
+{
+    __shared__ float px[kSumH + 7][kSumW + 8];
+    __shared__ double sq[kSumH + 7][kSumW];
+    const int x0 = blockIdx.x * kSumW, y0 = blockIdx.y * kSumH;
+    for (int i = threadIdx.x; i < (kSumH + 7) * (kSumW + 8); i += 256) {
+        const int r = i / (kSumW + 8), c = i - r * (kSumW + 8);
+        px[r][c] = src[(long long)min(y0 + r, height - 1) * pitch + min(x0 + c, width - 1)];
+    }
+    __syncthreads();
+    const int c = threadIdx.x & 63;
+    for (int r = threadIdx.x >> 6; r < kSumH + 7; r += 4) {
+        double s = 0.0, q = 0.0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const double v = double(px[r][c + j]);
+            s += v;
+            q = __builtin_fma(v, v, q);
+        }
+        sq[r][c] = q;
+        if (r < kSumH && y0 + r < height && x0 + c < width) {
+            float *out = hb + (long long)(y0 + r) * hpitch + x0 + c;
+            out[0] = px[r][c];
+            if (x0 + c <= width - 8) {
+                out[hplane] = float(s);
+            }
+        }
+    }
+    __syncthreads();
+    for (int r = threadIdx.x >> 6; r < kSumH; r += 4) {
+        double b = 0.0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            b += sq[r + i][c];
+        }
+        if (y0 + r <= height - 8 && x0 + c <= width - 8) {
+            hb[2 * hplane + (long long)(y0 + r) * hpitch + x0 + c] = float(b);
+        }
+    }
+}
+
 template <int CM, bool EXACT>
 __global__ __launch_bounds__(256) void bm3d_match(MatchArgs A)
 {
@@ -3288,12 +3848,30 @@ static hipError_t launch_temporal(const MatchArgs &a, int fp_mode, hipStream_t s
                : geo == 7 ? go(bm3d_match_predictive<kFpExplicit, 2, 7>)
                           : go(bm3d_match_predictive<kFpExplicit, 0, 0>);
     }
+    if (a.hb) {
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, block, 0, s, a);
+            return hipGetLastError();
+        };
+        if (a.ps_range > 7) {
+            return fused ? go(bm3d_match_steps<kFpAll, 32>) : go(bm3d_match_steps<kFpExplicit, 32>);
+        }
+        return fused ? go(bm3d_match_steps<kFpAll, 16>) : go(bm3d_match_steps<kFpExplicit, 16>);
+    }
     const size_t tlds = size_t(temporal_lds_bytes(a.t_rows, a.ps_range));
     if (fused) {
         hipLaunchKernelGGL((bm3d_match<kFpAll, false>), grid, block, tlds, s, a);
     } else {
         hipLaunchKernelGGL((bm3d_match<kFpExplicit, false>), grid, block, tlds, s, a);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_sum_planes(const float *src, int pitch, int width, int height, float *hb, int hb_pitch,
+                             long long hb_plane, hipStream_t s)
+{
+    const dim3 grid((width + kSumW - 1) / kSumW, (height + kSumH - 1) / kSumH);
+    hipLaunchKernelGGL(bm3d_sum_planes, grid, dim3(256), 0, s, src, pitch, width, height, hb, hb_plane, hb_pitch);
     return hipGetLastError();
 }
 
