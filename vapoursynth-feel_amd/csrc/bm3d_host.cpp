@@ -1369,12 +1369,18 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
             hipSuccess) {
             return dev_fail(e, "hipMemcpy");
         }
-        if (d.radius > 0 && 2 * d.radius * d.ps_num >= 8) {
+        const int insertions = 2 * d.radius * d.ps_num;
+        if (insertions >= 8 || (insertions >= 4 && d.nref >= 128 * kComputeUnits)) {
             // binning pays where a group takes at least 8 temporal
-            // insertions (at 4K, radius 1, ps_num 2 the gather cost more
-            // than the atomics it replaced); a group holds at most 7
-            // other-frame blocks (the self block is always a member);
-            // binning is skipped where its records would take more than 4 GiB
+            // insertions, with 4 to 7 on frames of many blocks, where the
+            // gather's time is no longer its launch and the atomics' is their
+            // traffic (radius 1, ps_num 2: 3840x2160, block_step 4, estimate
+            // 973 us with atomics, 648 and a gather of 150 without, the frame
+            // 3.0 ms and 2.8; 825x532, 27 k blocks, 64 us, 43 and 17;
+            // 1280x720, block_step 8, 14 k, 53 us, 48 and 14); a group holds
+            // at most 7 other-frame blocks (the self block is always a
+            // member); binning is skipped where its records would take more
+            // than 4 GiB
             const long long tiles = (long long)d.tiles_x * d.tiles_y;
             const long long per_tile = (long long)d.tile_bx * d.tile_by * 7;
             const long long rec_bytes = tiles * per_tile * 256;
