@@ -74,8 +74,8 @@ struct MatchArgs {
     // layout (column-major source region, per-block distance rows)
     int run_blocks, runs_x;
     int region_cols, region_rows, dist_cols;
-    // nonzero: bm3d_match_cols with runs of that many grid rows instead
-    int cols_vb;
+    // nonzero: bm3d_match_cols (runs of two grid rows) instead
+    int use_cols;
     // temporal search after bm3d_match_rows: distance rows per wavefront
     // (ps_num * (2 ps_range + 1)) for the threshold selection, 0: list
     int t_rows;

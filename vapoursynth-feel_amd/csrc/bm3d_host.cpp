@@ -228,7 +228,7 @@ struct Instance {
     // workgroup run and the LDS layout; run_blocks == 0 selects the
     // per-wavefront search instead
     int run_blocks = 0, runs_x = 0, region_cols = 0, region_rows = 0, dist_cols = 0;
-    int cols_vb = 0;             // grid rows per run of bm3d_match_cols (0: bm3d_match_rows)
+    int use_cols = 0;            // spatial search by bm3d_match_cols (0: bm3d_match_rows)
     int pred_pair = 0;           // temporal search: both directions per wavefront
     int t_rows = 0;  // temporal threshold selection: distance rows per wavefront (0: list)
     float *dst_dev = nullptr;    // one plane
@@ -630,7 +630,7 @@ struct Instance {
         m.region_cols = region_cols;
         m.region_rows = region_rows;
         m.dist_cols = dist_cols;
-        m.cols_vb = cols_vb;
+        m.use_cols = use_cols;
         m.t_rows = t_rows;
         m.pred_pair = pred_pair;
         m.hb = lane_hb();
@@ -1126,16 +1126,15 @@ std::string parse_args(const vsfeel_bm3d_args &a, Instance &d)
                 d.dist_cols = dcols;
             }
         }
-        // bm3d_match_cols where it was compiled and the frame holds its run's
-        // region, of two grid rows where that leaves two workgroups for every
-        // compute unit
-        for (int vb = 2; vb >= 1 && d.run_blocks > 0 && d.cols_vb == 0; --vb) {
-            const ColsGeometry g = cols_geometry(16, 4, vb);
-            if (d.bm_range == 16 && d.block_step == 4 && d.width >= g.rcols && d.height >= g.rrows &&
-                (vb == 1 || (d.nx + g.nb - 1) / g.nb * ((d.ny + 1) / 2) >= 2 * kComputeUnits)) {
-                d.cols_vb = vb;
-            }
-        }
+        // bm3d_match_cols where it was compiled, the frame holds its run's
+        // region and there are blocks enough to hide the exact search of the
+        // runs without noise, which few blocks wait for (cartoon 428x316: 43
+        // us by rows, 61 by columns; 853x481, 25 k blocks: noisy 65 and 55,
+        // cartoon 78 and 84; 1280x720, 57 k: 128 and 97, 135 and 142;
+        // 1920x1080: 261 and 198, 284 and 261)
+        const ColsGeometry g = cols_geometry(16, 4, 2);
+        d.use_cols = d.run_blocks > 0 && d.bm_range == 16 && d.block_step == 4 && d.width >= g.rcols &&
+                     d.height >= g.rrows && d.nref >= 128 * kComputeUnits;
         if (d.run_blocks > 0 && d.radius > 0) {
             // the predictive search's rows of one step, one per lane
             const int wh = 2 * d.ps_range + 1;

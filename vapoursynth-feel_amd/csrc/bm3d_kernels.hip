@@ -3908,18 +3908,15 @@ hipError_t launch_match(const MatchArgs &a, int fp_mode, hipStream_t s, bool tem
         // geometry they were slower (778x751, bm_range 12 at block_step 8:
         // 43 us against 24), compiled for bm_range 9 not faster (640x360 at
         // block_step 8: 18 against 17 us; 512x512 at 4: 23 against 27 us)
-        if (a.cols_vb > 0) {
-            auto cols = [&](auto kernel, int vb) {
-                const ColsGeometry g = cols_geometry(16, 4, vb);
+        if (a.use_cols) {
+            auto cols = [&](auto kernel) {
+                const ColsGeometry g = cols_geometry(16, 4, 2);
                 const size_t clds = size_t(cols_layout(g).total) * sizeof(float);
-                const dim3 cgrid(((a.ny + vb - 1) / vb) * ((a.nx + g.nb - 1) / g.nb));
+                const dim3 cgrid(((a.ny + 1) / 2) * ((a.nx + g.nb - 1) / g.nb));
                 hipLaunchKernelGGL(kernel, cgrid, block, clds, s, rows);
                 return hipGetLastError();
             };
-            if (a.cols_vb == 2) {
-                return fused ? cols(bm3d_match_cols<kFpAll, 16, 4, 2>, 2) : cols(bm3d_match_cols<kFpExplicit, 16, 4, 2>, 2);
-            }
-            return fused ? cols(bm3d_match_cols<kFpAll, 16, 4, 1>, 1) : cols(bm3d_match_cols<kFpExplicit, 16, 4, 1>, 1);
+            return fused ? cols(bm3d_match_cols<kFpAll, 16, 4, 2>) : cols(bm3d_match_cols<kFpExplicit, 16, 4, 2>);
         }
         const size_t lds = size_t(rows_lds_bytes(a.region_cols, a.region_rows, a.run_blocks, a.dist_cols));
         const dim3 rgrid(a.ny * a.runs_x);
