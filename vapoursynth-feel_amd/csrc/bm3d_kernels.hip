@@ -3623,6 +3623,8 @@ __global__ __launch_bounds__(256) void bm3d_gather(GatherArgs A)
 // tile order.  Where every pixel lies in at most 3 x 3 tiles (span3) all of
 // a pixel's loads are issued before the first add (absent tiles add +0.0f,
 // which leaves the sum's bits unchanged), with 32-bit offsets.
+// SPAN3: at most 3 x 3 tiles over any pixel
+template <bool SPAN3>
 __global__ __launch_bounds__(256) void bm3d_tile_reduce(ReduceArgs A)
 {
     const int x = blockIdx.x * 64 + (threadIdx.x & 63);
@@ -3633,7 +3635,7 @@ __global__ __launch_bounds__(256) void bm3d_tile_reduce(ReduceArgs A)
     const int2 cr = A.col_tiles[x];
     const int2 rr = A.row_tiles[y];
     float wd = 0.0f, wt = 0.0f;
-    if (A.span3) {
+    if constexpr (SPAN3) {
         const uint32_t plane = uint32_t(A.region_h) * uint32_t(A.region_w);
         const int nty = rr.y - rr.x + 1, ntx = cr.y - cr.x + 1;
         float vd[9], vw[9];
@@ -3657,15 +3659,41 @@ __global__ __launch_bounds__(256) void bm3d_tile_reduce(ReduceArgs A)
             wt += vw[k];
         }
     } else {
+        // many tiles over a pixel (small frames: up to all of them): 8 at a
+        // time, their origins and then their values loaded together, added
+        // one by one in the tiles' order (52x54 at block_step 4, bm_range 20:
+        // 50 us with a load waited for per tile, 28 now; 80x44 at 4, 20: 48 us
+        // and 24; 203x157 at 4, 9: 10 and 7)
+        constexpr int kBatch = 12;
         const long long plane = (long long)A.region_h * A.region_w;
-        for (int ty = rr.x; ty <= rr.y; ++ty) {
-            const int ly = y - A.tile_y0[ty];
-            for (int tx = cr.x; tx <= cr.y; ++tx) {
-                const int lx = x - A.tile_x0[tx];
-                const float *t =
-                    A.scratch + (long long)(ty * A.tiles_x + tx) * 2 * plane + (long long)ly * A.region_w + lx;
-                wd += t[0];
-                wt += t[plane];
+        int ty = rr.x, tx = cr.x;
+        const int n = max(rr.y - rr.x + 1, 0) * max(cr.y - cr.x + 1, 0);
+        for (int i0 = 0; i0 < n; i0 += kBatch) {
+            int tile[kBatch], lx[kBatch], ly[kBatch];
+            float vd[kBatch], vw[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                tile[u] = ty * A.tiles_x + tx;
+                lx[u] = x - A.tile_x0[tx];
+                ly[u] = y - A.tile_y0[ty];
+                // (past the last tile: the last again)
+                const bool more = i0 + u + 1 < n, wrap = tx == cr.y;
+                ty += more && wrap ? 1 : 0;
+                tx = more ? (wrap ? cr.x : tx + 1) : tx;
+            }
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                vd[u] = vw[u] = 0.0f;
+                if (i0 + u < n) {
+                    const float *t = A.scratch + (long long)tile[u] * 2 * plane + (long long)ly[u] * A.region_w + lx[u];
+                    vd[u] = t[0];
+                    vw[u] = t[plane];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                wd += vd[u];
+                wt += vw[u];
             }
         }
     }
@@ -4006,7 +4034,11 @@ hipError_t launch_divide(const float *num, int num_pitch, const float *den, int 
 hipError_t launch_tile_reduce(const ReduceArgs &a, hipStream_t s)
 {
     const dim3 grid((a.width + 63) / 64, (a.height + 3) / 4), block(256);
-    hipLaunchKernelGGL(bm3d_tile_reduce, grid, block, 0, s, a);
+    if (a.span3) {
+        hipLaunchKernelGGL(bm3d_tile_reduce<true>, grid, block, 0, s, a);
+    } else {
+        hipLaunchKernelGGL(bm3d_tile_reduce<false>, grid, block, 0, s, a);
+    }
     return hipGetLastError();
 }
 
