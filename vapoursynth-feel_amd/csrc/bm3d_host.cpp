@@ -258,7 +258,8 @@ struct Instance {
     std::mutex mu;
 
     // process_device replays its launch sequence from a HIP graph while the
-    // call's arguments repeat (captured on the first call with new ones)
+    // call's arguments repeat (captured on the second call in a row with the
+    // same ones; last_key holds the last call's)
     struct GraphKey {
         const float *data, *ref;
         int64_t frame_stride, out_frame_stride;
@@ -274,7 +275,8 @@ struct Instance {
     bool graphs = true;            // process_device replays its graph
     bool request_graphs = false;   // get_frame launches from per-slot graphs
     hipGraphExec_t graph_exec = nullptr;
-    GraphKey graph_key{};
+    GraphKey graph_key{}, last_key{};
+    bool last_key_set = false;
     hipEvent_t fork_ev = nullptr, join_ev = nullptr;  // orders the instance stream with a null-stream caller
 
     // The host-buffer path (allocated on first use).  Requests overlap: a
@@ -1933,12 +1935,21 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
         }
         return e;
     };
-    if (d.graphs && !d.timing && count > 0) {
+    const Instance::GraphKey key{clip->data, clip->ref, clip->frame_stride, out_frame_stride,
+                                 clip->pitch, first, count, out_pitch, out};
+    // a launch sequence is captured when a call repeats the last one's
+    // arguments; others, such as those of a caller that allocates its output
+    // anew, are launched directly: capturing and instantiating costs more than
+    // the few launches it would save once (64x48, one frame, a new output
+    // every call: 91 us with a capture each, 47 launched)
+    const bool repeats = d.last_key_set && d.last_key == key;
+    d.last_key = key;
+    d.last_key_set = true;
+    const bool held = d.graph_exec && d.graph_key == key;
+    if (d.graphs && !d.timing && count > 0 && (held || repeats)) {
         // replay from a graph captured on the instance stream, ordered after
         // and before the caller's stream by events
-        const Instance::GraphKey key{clip->data, clip->ref, clip->frame_stride, out_frame_stride,
-                                     clip->pitch, first, count, out_pitch, out};
-        if (!d.graph_exec || !(d.graph_key == key)) {
+        if (!held) {
             // the previous graph, or host-buffer requests, may still run on
             // the instance stream: capture on an idle one
             VSFEEL_HIP(hipStreamSynchronize(d.stream), "hipStreamSynchronize");
