@@ -1378,10 +1378,14 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
             // traffic (radius 1, ps_num 2: 3840x2160, block_step 4, estimate
             // 973 us with atomics, 648 and a gather of 150 without, the frame
             // 3.0 ms and 2.8; 825x532, 27 k blocks, 64 us, 43 and 17;
-            // 1280x720, block_step 8, 14 k, 53 us, 48 and 14); a group holds
-            // at most 7 other-frame blocks (the self block is always a
-            // member); binning is skipped where its records would take more
-            // than 4 GiB
+            // 1280x720, block_step 8, 14 k, 53 us, 48 and 14).  How much
+            // depends on the motion, which decides how many of the blocks
+            // come from other frames: seven 3840x2160 clips moving by
+            // different parts of a pixel, 4 frames: 12.0 -> 10.7, 12.0 ->
+            // 10.8, 11.9 -> 11.3 ms, four with few such blocks 2 to 3 %
+            // slower.  A group holds at most 7 other-frame blocks (the self
+            // block is always a member); binning is skipped where its records
+            // would take more than 4 GiB
             const long long tiles = (long long)d.tiles_x * d.tiles_y;
             const long long per_tile = (long long)d.tile_bx * d.tile_by * 7;
             const long long rec_bytes = tiles * per_tile * 256;
