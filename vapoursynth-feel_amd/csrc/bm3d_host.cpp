@@ -650,8 +650,9 @@ struct Instance {
     }
 
     // forgets the frames whose sums the lanes hold: at the start and the end
-    // of everything but the host path, and after a failure there (what was
-    // enqueued may not have run)
+    // of everything but the host path (a replayed graph writes the planes, too,
+    // without passing match()), and after a failure there (what was enqueued
+    // may not have run)
     void forget_sums()
     {
         for (auto &l : hb_frame) {
@@ -1859,8 +1860,6 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
             Instance &d;
             ~LaneReset() { d.lane = 0; }
         } lane_reset{d};
-        // (the caller may rewrite the clip between calls)
-        d.forget_sums();
         Instance::SumsScope sums{d};
         std::vector<int> held(d.res_cap, -1);
         std::vector<int> slot_of(d.tw);
@@ -1950,6 +1949,12 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
     d.last_key = key;
     d.last_key_set = true;
     const bool held = d.graph_exec && d.graph_key == key;
+    // from here on, whether launched, captured or replayed, and also where one
+    // of these fails: the res slots and the planes of sums hold this call's
+    // frames, not the host path's (and the caller may rewrite the clip between
+    // calls)
+    std::fill(d.res_frame.begin(), d.res_frame.end(), -1);
+    d.forget_sums();
     if (d.graphs && !d.timing && count > 0 && (held || repeats)) {
         // replay from a graph captured on the instance stream, ordered after
         // and before the caller's stream by events
@@ -1993,8 +1998,6 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
     } else {
         VSFEEL_HIP(enqueue(s), "launch");
     }
-    // the res slots now hold this call's stacks, not the host path's frames
-    std::fill(d.res_frame.begin(), d.res_frame.end(), -1);
     VSFEEL_HIP(d.end_on(s), "hipEventRecord");
     return VSFEEL_BM3D_OK;
 }
