@@ -760,21 +760,24 @@ __global__ __launch_bounds__(256) void bm3d_match_rows(MatchArgs A)
 // / 0.323, without noise 0.248 / 0.277, texture along columns 0.247 / 0.247.
 // ---------------------------------------------------------------------------
 
-// |D~ - D| <= kEps (N + box) for the candidate, where N = sum_j |c_j|^2 +
-// 8 |c7|^2 bounds every |R_k|^2: with u = 2^-24, the centring costs 4u (N +
+// |D~ - D| <= kEps (N + box) + kTiny for the candidate, where N = sum_j |c_j|^2
+// + 8 |c7|^2 bounds every |R_k|^2: with u = 2^-24, the centring costs 4u (N +
 // box), h 3u N + 3u box, box 7u box, |R_k|^2 16u N, the correction's 7 chains
 // of 8 and their sums 30u N + 45u box, the main chain 27u N + 36u box and the
-// FP32 distance itself 24u (N + box): below 2^7 u = 2^-17 of N + box.
-// sqrt(box) <= sqrt(|R_k|^2) + sqrt(D) turns that into 3 kEps N + 2 kEps D.
-// Keys hold D~ + 4 kEps N, which is never negative.  With T the 8th smallest
-// of these (or an upper bound of it), 8 candidates have D <= T (1 + 3 kEps),
-// so the 8 nearest have D~ + 4 kEps N up to T (1 + 6 kEps) + 7 kEps N, which
-// select_threshold rounds up.
-constexpr float kEps = 0x1p-17f;
+// FP32 distance itself 24u (N + box): below 2^7 u = 2^-17 of N + box.  Below
+// 2^-126 each of the fewer than 300 products loses up to 2^-150 instead
+// (additions lose nothing there): kTiny covers those many times over.
+// sqrt(box) <= sqrt(|R_k|^2) + sqrt(D) turns that into 3 kEps N + 2 kEps D +
+// kTiny.  Keys hold D~ + 4 kEps N + kTiny, which is never negative.  With T the
+// 8th smallest of these (or an upper bound of it), 8 candidates have D <= T (1 +
+// 3 kEps), so the 8 nearest have D~ + 4 kEps N + kTiny up to T (1 + 6 kEps) +
+// 7 kEps N + 2 kTiny, which select_threshold rounds up.
+constexpr float kEps = 0x1p-17f, kTiny = 0x1p-126f;
+__device__ __forceinline__ float key_offset(float n) { return n * (4.0f * kEps) + kTiny; }
 __device__ __forceinline__ uint32_t select_threshold(uint32_t tk, float n)
 {
     const float t = __uint_as_float(tk);
-    return __float_as_uint(t + (t * 0x1p-13f + n * (8.0f * kEps)));
+    return __float_as_uint(t + (t * 0x1p-13f + (n * (8.0f * kEps) + 4.0f * kTiny)));
 }
 // runs with pixels whose squares' 8-column sum is not below this (huge or
 // non-finite ones) are searched exactly; below it nothing here overflows
@@ -1433,7 +1436,7 @@ __global__ __launch_bounds__(256, 3) void bm3d_match_cols(MatchArgs A)
         auto base_of = [&](int v) {
             const float *cn = cnorm + v * per + b * 8;
             const float n7 = cn[7];
-            return j < 7 ? cn[j] - n7 : 8.0f * n7 + norm_bound(cn) * (4.0f * kEps);
+            return j < 7 ? cn[j] - n7 : 8.0f * n7 + key_offset(norm_bound(cn));
         };
         // (of the centred columns, whose rounding the bound counts)
         auto coef_of = [&](const float *cb) { return -2.0f * ((cb[j] - m) - (cb[7] - m)); };
@@ -1689,7 +1692,7 @@ __global__ __launch_bounds__(256, 3) void bm3d_match_cols(MatchArgs A)
             const float *cf = coef + bl * 8;
             const float *cb = src + (y - ry0) * SS + (xb - rx0);
             const float *sp0 = src + (top - ry0) * SS + (left - rx0);
-            const float nr0 = 8.0f * cn[7] + n * (4.0f * kEps);
+            const float nr0 = 8.0f * cn[7] + key_offset(n);
             float c7[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
