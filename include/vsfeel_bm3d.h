@@ -256,8 +256,10 @@ int vsfeel_bm3d_kernel_times(vsfeel_bm3d *h, double *ms, int64_t *count);
  * radius > 0, tile reduction, aggregation) into a HIP graph on the
  * instance's stream when a call's arguments are those of the call before it,
  * and later calls with identical arguments replay it, ordered after and
- * before the caller's stream by events; other calls launch directly.  (At
- * radius > 0
+ * before the caller's stream by events; other calls launch directly.  A
+ * sequence on several lanes (several frames, or any at radius > 0) is
+ * captured only as the handle's first graph, which then stays: other
+ * arguments launch directly from there on.  (At radius > 0
  * the replayed graph ran the two lanes' cross-linked branches with less
  * overlap than direct launches: 980 against 1024 frames/s at 1080p radius
  * 2, hence the default there.)  Bit 1:

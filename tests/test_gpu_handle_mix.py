@@ -11,9 +11,10 @@ pytestmark = pytest.mark.gpu
 KW = dict(sigma=3.0, block_step=2, bm_range=5, ps_num=3, ps_range=7, extractor_exp=2)
 
 
-@pytest.mark.parametrize("graphs", [0, 1])
+# (lanes, graphs): launched; captured and replayed on two lanes and on one
+@pytest.mark.parametrize("lanes,graphs", [(None, 0), (None, 1), (1, 1)])
 @pytest.mark.parametrize("radius", [1, 2])
-def test_requests_after_device_calls_of_another_clip(radius, graphs):
+def test_requests_after_device_calls_of_another_clip(radius, lanes, graphs, monkeypatch):
     import torch
     if not torch.cuda.is_available():
         pytest.skip("no HIP device")
@@ -25,6 +26,8 @@ def test_requests_after_device_calls_of_another_clip(radius, graphs):
     fresh = BM3Dv2(Clip.gray(host), radius=radius, **KW)
     want = [fresh.get_frame(i)[0] for i in range(n)]
 
+    if lanes is not None:
+        monkeypatch.setenv("VSFEEL_BM3D_LANES", str(lanes))
     node = BM3Dv2(Clip.gray(host), radius=radius, **KW)
     L = _lib.load()
     assert L.vsfeel_bm3d_set_graphs(node._handle, graphs) == _lib.OK
@@ -41,8 +44,8 @@ def test_requests_after_device_calls_of_another_clip(radius, graphs):
         assert rc == _lib.OK, err.value
         return out.cpu().numpy()
 
-    first = process()  # launched
-    assert np.array_equal(process(), first)  # captured and replayed (graphs 1)
+    first = process()
+    assert np.array_equal(process(), first)
     for m in (5, 6, 4, 0, 8):
         got = node.get_frame(m)[0]
         assert np.array_equal(got, want[m]), f"frame {m} differs by {float(np.abs(got - want[m]).max())}"

@@ -277,6 +277,7 @@ struct Instance {
     hipGraphExec_t graph_exec = nullptr;
     GraphKey graph_key{}, last_key{};
     bool last_key_set = false;
+    bool captured = false, captured_forks = false;  // a graph was captured; one that forks lanes
     hipEvent_t fork_ev = nullptr, join_ev = nullptr;  // orders the instance stream with a null-stream caller
 
     // The host-buffer path (allocated on first use).  Requests overlap: a
@@ -1855,6 +1856,8 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
     // end.
     const int nlanes = d.timing ? 1 : d.lanes;
     const bool fused = d.fuses();
+    // whether lanes run on side streams (at radius 0 lane 0 is the launch stream)
+    const bool forks = nlanes > 1 && (!fused || count > 1);
     auto enqueue = [&](hipStream_t q) -> hipError_t {
         struct LaneReset {
             Instance &d;
@@ -1869,7 +1872,7 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
         auto side = [&](int j) { return nlanes == 1 ? -1 : fused ? j - 1 : j; };
         auto lane_stream = [&](int j) { return side(j) < 0 ? q : d.stream_l[side(j)]; };
         hipError_t e = hipSuccess;
-        if (nlanes > 1) {
+        if (forks) {
             e = hipEventRecord(d.lane_fork, q);
         }
         int k = 0;
@@ -1944,7 +1947,13 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
     // arguments; others, such as those of a caller that allocates its output
     // anew, are launched directly: capturing and instantiating costs more than
     // the few launches it would save once (64x48, one frame, a new output
-    // every call: 91 us with a capture each, 47 launched)
+    // every call: 91 us with a capture each, 47 launched).  A sequence that
+    // forks lanes is captured only as the handle's first graph, and nothing
+    // after it: capturing one again with the graph before it destroyed has
+    // ended in a segmentation fault of the host whose cause is not known.
+    // Later arguments launch, which is no slower by much (8 frames of 640x360:
+    // one handle 231 us replayed, 201 launched; three handles in turn 227 and
+    // 238)
     const bool repeats = d.last_key_set && d.last_key == key;
     d.last_key = key;
     d.last_key_set = true;
@@ -1955,7 +1964,8 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
     // calls)
     std::fill(d.res_frame.begin(), d.res_frame.end(), -1);
     d.forget_sums();
-    if (d.graphs && !d.timing && count > 0 && (held || repeats)) {
+    const bool capturable = !d.captured || (!forks && !d.captured_forks);
+    if (d.graphs && !d.timing && count > 0 && (held || (repeats && capturable))) {
         // replay from a graph captured on the instance stream, ordered after
         // and before the caller's stream by events
         if (!held) {
@@ -1971,6 +1981,8 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
                 (void)hipGraphExecDestroy(d.graph_exec);
                 d.graph_exec = nullptr;
             }
+            d.captured = true;
+            d.captured_forks = forks;
             VSFEEL_HIP(hipStreamBeginCapture(d.stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
             const hipError_t e = enqueue(d.stream);
             hipGraph_t g = nullptr;
