@@ -79,3 +79,31 @@ def test_other_calls_leave_a_held_graph(calls, counts):
     # one frame or several (captured), then several or one (launched), then the first again
     sequence = [["create", 96, 80, 5, SPATIAL]] + [["process", "A", 0, n] for n in counts]
     assert _kinds(calls(sequence)[1:]) == ["direct", "capture", "direct", "direct", "direct", "replay"]
+
+
+# 2 radius ps_num insertions: as many as always bin, and few on a frame of 32768 blocks and more
+@pytest.mark.parametrize("w,h,kw", [
+    (120, 104, dict(sigma=3.0, block_step=4, bm_range=5, radius=2, ps_num=2, ps_range=4)),
+    (376, 361, dict(sigma=3.0, block_step=2, bm_range=3, radius=1, ps_num=2, ps_range=4)),
+])
+def test_no_room_for_the_bins_leaves_the_atomic_scatter(calls, w, h, kw):
+    def run(limit):
+        return calls([["limit", limit], ["create", w, h, 3, kw], ["process", "A", 0, 3], ["free"]])[1:]
+
+    def bins(result):
+        return any("bm3d_gather" in line for line in result[1]["log"])
+
+    roomy = run(1 << 50)
+    assert roomy[0]["rc"] == roomy[1]["rc"] == 0 and bins(roomy)
+    everything = roomy[0]["live"]
+    # the records of a lane: 64 floats for each of 7 blocks of every group
+    ny, nx = (h - 8 + kw["block_step"] - 1) // kw["block_step"] + 1, (w - 8 + kw["block_step"] - 1) // kw["block_step"] + 1
+    records = nx * ny * 7 * 64 * 4
+    assert everything > 2 * records
+    for limit in (everything - 1, everything - records, everything - records - 1, everything - 2 * records):
+        tight = run(limit)
+        assert tight[0]["rc"] == tight[1]["rc"] == 0, (limit, everything)
+        assert not bins(tight) and any("bm3d_estimate" in line for line in tight[1]["log"])
+        # what was made before one of them failed is given back
+        assert tight[0]["live"] <= everything - 2 * records
+        assert tight[2]["live"] == 0

@@ -495,6 +495,22 @@ struct Instance {
         return e;
     }
 
+    // the binning's buffers of every lane: the atomic path needs none
+    void free_bins()
+    {
+        for (int i = 0; i < kMaxLanes; ++i) {
+            float *&r = i ? rec_l[i - 1] : rec;
+            uint32_t *&c = i ? cell_count_l[i - 1] : cell_count;
+            uint2 *&l = i ? cell_list_l[i - 1] : cell_list;
+            (void)hipFree(r);
+            (void)hipFree(c);
+            (void)hipFree(l);
+            r = nullptr;
+            c = nullptr;
+            l = nullptr;
+        }
+    }
+
     ~Instance()
     {
         if (device < 0) {
@@ -520,9 +536,7 @@ struct Instance {
         (void)hipFree(scratch);
         (void)hipFree(origins);
         (void)hipFree(tile_tables);
-        (void)hipFree(rec);
-        (void)hipFree(cell_count);
-        (void)hipFree(cell_list);
+        free_bins();
         (void)hipFree(psets);
         for (float *p : hb_l) {
             (void)hipFree(p);
@@ -533,9 +547,6 @@ struct Instance {
             (void)hipFree(psets_l[i]);
             (void)hipFree(spatial_l[i]);
             (void)hipFree(origins_l[i]);
-            (void)hipFree(rec_l[i]);
-            (void)hipFree(cell_count_l[i]);
-            (void)hipFree(cell_list_l[i]);
             (void)hipFree(dst_l[i]);
             if (lane_join[i]) {
                 (void)hipEventDestroy(lane_join[i]);
@@ -1387,7 +1398,7 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
             // 10.8, 11.9 -> 11.3 ms, four with few such blocks 2 to 3 %
             // slower.  A group holds at most 7 other-frame blocks (the self
             // block is always a member); binning is skipped where its records
-            // would take more than 4 GiB
+            // would take more than 4 GiB, or find no room
             const long long tiles = (long long)d.tiles_x * d.tiles_y;
             const long long per_tile = (long long)d.tile_bx * d.tile_by * 7;
             const long long rec_bytes = tiles * per_tile * 256;
@@ -1412,12 +1423,6 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
                     d.cell_cap = std::min(std::max(std::atoi(cap), 1), 4096);
                 }
                 d.cell_count_elems = (2LL * d.radius * d.ncells + 63) / 64 * 64;
-                if ((e = hipMalloc(&d.rec, size_t(tiles * per_tile) * 64 * sizeof(float))) != hipSuccess ||
-                    (e = hipMalloc(&d.cell_count, size_t(d.cell_count_elems) * sizeof(uint32_t))) != hipSuccess ||
-                    (e = hipMalloc(&d.cell_list, size_t(2LL * d.radius * d.ncells * d.cell_cap) * sizeof(uint2))) !=
-                        hipSuccess) {
-                    return dev_fail(e, "hipMalloc");
-                }
             }
         }
         // VSFEEL_BM3D_LANES caps the lanes (1: one stream and no extra
@@ -1433,7 +1438,6 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
             // linked branches less than direct launches do (980 against 1024
             // frames/s at 1080p radius 2): launch directly by default
             d.graphs = d.radius == 0;
-            const size_t rec_bytes = size_t((long long)d.tiles_x * d.tiles_y * d.rec_per_tile) * 64 * sizeof(float);
             if ((e = hipEventCreateWithFlags(&d.lane_fork, hipEventDisableTiming)) != hipSuccess) {
                 return dev_fail(e, "hipEventCreate");
             }
@@ -1465,15 +1469,25 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
                      (e = hipMalloc(&d.psets_l[i], size_t(d.pset_bytes))) != hipSuccess) ||
                     (d.spatial && (e = hipMalloc(&d.spatial_l[i], size_t(d.nref) * 8 * sizeof(uint2))) != hipSuccess) ||
                     (d.origins && (e = hipMalloc(&d.origins_l[i], plane * 2 * d.radius)) != hipSuccess) ||
-                    (d.rec && (e = hipMalloc(&d.rec_l[i], rec_bytes)) != hipSuccess) ||
-                    (d.rec && (e = hipMalloc(&d.cell_count_l[i], size_t(d.cell_count_elems) * sizeof(uint32_t))) !=
-                                  hipSuccess) ||
-                    (d.rec && (e = hipMalloc(&d.cell_list_l[i],
-                                             size_t(2LL * d.radius * d.ncells * d.cell_cap) * sizeof(uint2))) !=
-                                  hipSuccess) ||
                     (d.radius == 0 && (e = hipMalloc(&d.dst_l[i], plane)) != hipSuccess)) {
                     return dev_fail(e, "hipMalloc");
                 }
+            }
+        }
+    }
+    // the binning's buffers after everything that a call cannot do without:
+    // where one of them finds no room, the blocks go down the atomic path
+    if (d.rec_per_tile > 0) {
+        const size_t rec_bytes = size_t((long long)d.tiles_x * d.tiles_y * d.rec_per_tile) * 64 * sizeof(float);
+        const size_t count_bytes = size_t(d.cell_count_elems) * sizeof(uint32_t);
+        const size_t list_bytes = size_t(2LL * d.radius * d.ncells * d.cell_cap) * sizeof(uint2);
+        for (int i = 0; i < d.lanes; ++i) {
+            if (hipMalloc(i ? &d.rec_l[i - 1] : &d.rec, rec_bytes) != hipSuccess ||
+                hipMalloc(i ? &d.cell_count_l[i - 1] : &d.cell_count, count_bytes) != hipSuccess ||
+                hipMalloc(i ? &d.cell_list_l[i - 1] : &d.cell_list, list_bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                d.free_bins();
+                break;
             }
         }
     }
