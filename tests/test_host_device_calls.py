@@ -107,3 +107,28 @@ def test_no_room_for_the_bins_leaves_the_atomic_scatter(calls, w, h, kw):
         # what was made before one of them failed is given back
         assert tight[0]["live"] <= everything - 2 * records
         assert tight[2]["live"] == 0
+
+
+def test_no_room_for_the_sums_leaves_the_search_without_them(calls):
+    # 3 windows of 15 rows on 2448 blocks and more, searched with planes of sums
+    w, h = 120, 104
+    kw = dict(sigma=3.0, block_step=2, bm_range=5, radius=1, ps_num=3, ps_range=7)
+
+    def run(limit):
+        return calls([["limit", limit], ["create", w, h, 3, kw], ["process", "A", 0, 3], ["free"]])[1:]
+
+    def sums(result):
+        return any("bm3d_sum_planes" in line for line in result[1]["log"])
+
+    roomy = run(1 << 50)
+    assert roomy[0]["rc"] == roomy[1]["rc"] == 0 and sums(roomy)
+    everything = roomy[0]["live"]
+    # a lane's: 3 planes for each of 3 frames, rows of a multiple of 16 floats, 40 rows past the frame
+    planes = 3 * 3 * ((w + 15) // 16 * 16) * (h + 40) * 4
+    needed = everything - 2 * planes
+    for limit in (everything - 1, everything - planes, everything - planes - 1, needed + planes // 2, needed):
+        tight = run(limit)
+        assert tight[0]["rc"] == tight[1]["rc"] == 0, (limit, everything)
+        assert sums(tight) == (limit >= needed + planes)
+        assert any("bm3d_match" in line for line in tight[1]["log"])
+        assert tight[2]["live"] == 0

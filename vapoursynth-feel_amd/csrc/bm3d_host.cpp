@@ -1321,16 +1321,6 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
         (e = hipMalloc(&d.dst_dev, plane)) != hipSuccess) {
         return dev_fail(e, "hipMalloc");
     }
-    // (without the room the search that needs none is taken)
-    auto alloc_sums = [&](int lane) {
-        if (d.hb_plane > 0 &&
-            hipMalloc(&d.hb_l[lane], size_t(d.hb_plane) * 3 * d.tw * sizeof(float)) != hipSuccess) {
-            d.hb_l[lane] = nullptr;
-            (void)hipGetLastError();
-        }
-    };
-    alloc_sums(0);
-    d.forget_sums();
     if (d.operand != kOperandFp32) {
         d.pset_bytes = (plane_set_bytes(d.width, d.height) + 255) & ~255LL;
         if ((e = hipMalloc(&d.psets, size_t(d.pset_bytes))) != hipSuccess) {
@@ -1462,7 +1452,6 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
                 }
             }
             for (int i = 0; i < d.lanes - 1; ++i) {
-                alloc_sums(i + 1);
                 if ((e = hipMalloc(&d.groups_l[i], size_t(d.nref) * 8 * sizeof(uint32_t))) != hipSuccess ||
                     (e = hipMalloc(&d.scratch_l[i], scratch_elems * sizeof(float))) != hipSuccess ||
                     (d.operand != kOperandFp32 &&
@@ -1491,6 +1480,15 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
             }
         }
     }
+    // then the planes of sums: without the room for a lane's, its search is the
+    // one that needs none
+    for (int i = 0; i < d.lanes && d.hb_plane > 0; ++i) {
+        if (hipMalloc(&d.hb_l[i], size_t(d.hb_plane) * 3 * d.tw * sizeof(float)) != hipSuccess) {
+            d.hb_l[i] = nullptr;
+            (void)hipGetLastError();
+        }
+    }
+    d.forget_sums();
     d.src_frame.assign(d.src_ring, -1);
     d.res_frame.assign(d.res_cap, -1);
     *out = h;
