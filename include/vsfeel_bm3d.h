@@ -250,19 +250,15 @@ int vsfeel_bm3d_kernel_times(vsfeel_bm3d *h, double *ms, int64_t *count);
 
 /*
  * Graph launches; `enable` is a bit set (default 1 at radius 0, 0 at
- * radius > 0 where process_device runs two lanes).  Bit 0:
- * vsfeel_bm3d_process_device captures its launch sequence (per output frame:
- * slot clears, matching, filtering, the other frames' sums and weights at
- * radius > 0, tile reduction, aggregation) into a HIP graph on the
- * instance's stream when a call's arguments are those of the call before it,
- * and later calls with identical arguments replay it, ordered after and
- * before the caller's stream by events; other calls launch directly.  A
- * sequence on several lanes (several frames, or any at radius > 0) is
- * captured only as the handle's first graph, which then stays: other
- * arguments launch directly from there on.  (At radius > 0
- * the replayed graph ran the two lanes' cross-linked branches with less
- * overlap than direct launches: 980 against 1024 frames/s at 1080p radius
- * 2, hence the default there.)  Bit 1:
+ * radius > 0).  Bit 0: calls of vsfeel_bm3d_process_device that run on one
+ * lane (one frame at radius 0; any call of a handle made with
+ * VSFEEL_BM3D_LANES=1) capture their launch sequence (per output frame: slot
+ * clears, matching, filtering, the other frames' sums and weights at radius
+ * > 0, tile reduction, aggregation) into a HIP graph on the instance's
+ * stream when a call's arguments are those of the call before it, and later
+ * calls with identical arguments replay it, ordered after and before the
+ * caller's stream by events; other calls launch directly, those on several
+ * lanes always.  Bit 1:
  * vsfeel_bm3d_get_frame launches a request's kernels as one graph per
  * output slot and recompute pattern (the number of estimates the request
  * runs), captured on an idle stream and updated in place

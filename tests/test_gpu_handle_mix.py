@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 KW = dict(sigma=3.0, block_step=2, bm_range=5, ps_num=3, ps_range=7, extractor_exp=2)
 
 
-# (lanes, graphs): launched; captured and replayed on two lanes and on one
+# (lanes, graphs): a call on two lanes launches, one on one lane is captured and replayed
 @pytest.mark.parametrize("lanes,graphs", [(None, 0), (None, 1), (1, 1)])
 @pytest.mark.parametrize("radius", [1, 2])
 def test_requests_after_device_calls_of_another_clip(radius, lanes, graphs, monkeypatch):

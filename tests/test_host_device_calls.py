@@ -55,14 +55,11 @@ TEMPORAL = dict(SPATIAL, radius=1)
 @pytest.mark.parametrize("frames,first,count,kw", [
     (5, 0, 5, SPATIAL), (5, 1, 2, SPATIAL), (5, 0, 5, TEMPORAL), (5, 2, 1, TEMPORAL), (1, 0, 1, TEMPORAL),
 ])
-def test_calls_on_several_lanes_are_captured_once(calls, frames, first, count, kw):
-    # (capturing such a sequence again after other arguments has ended in a segmentation fault)
+def test_calls_on_several_lanes_are_never_captured(calls, frames, first, count, kw):
+    # (a capture after such a graph was destroyed has ended in a segmentation fault)
     sequence = [["create", 96, 80, frames, kw], ["set_graphs", 1]]
     sequence += [["process", out, first, count] for out in "AABBBAA"]
-    sequence += [["set_graphs", 0], ["set_graphs", 1]] + [["process", out, first, count] for out in "AAABB"]
-    got = calls(sequence)
-    assert _kinds(got[2:9]) == ["direct", "capture"] + ["direct"] * 3 + ["replay"] * 2
-    assert _kinds(got[11:]) == ["direct"] * 5
+    assert _kinds(calls(sequence)[2:]) == ["direct"] * 7
 
 
 @pytest.mark.parametrize("frames,count,kw,lanes", [(1, 1, SPATIAL, None), (5, 1, SPATIAL, None), (5, 5, SPATIAL, 1),
@@ -74,10 +71,9 @@ def test_calls_on_one_lane_replay_when_repeated(calls, frames, count, kw, lanes)
     assert got == ["direct", "capture", "replay", "direct", "replay", "direct", "capture"]
 
 
-@pytest.mark.parametrize("counts", [(1, 1, 5, 5, 5, 1), (5, 5, 1, 1, 1, 5)])
-def test_other_calls_leave_a_held_graph(calls, counts):
-    # one frame or several (captured), then several or one (launched), then the first again
-    sequence = [["create", 96, 80, 5, SPATIAL]] + [["process", "A", 0, n] for n in counts]
+def test_other_calls_leave_a_held_graph(calls):
+    # one frame (captured), then several (launched), then the frame again
+    sequence = [["create", 96, 80, 5, SPATIAL]] + [["process", "A", 0, n] for n in (1, 1, 5, 5, 5, 1)]
     assert _kinds(calls(sequence)[1:]) == ["direct", "capture", "direct", "direct", "direct", "replay"]
 
 

@@ -257,9 +257,9 @@ struct Instance {
     std::vector<int> res_frame;  // frame whose estimate stack each res slot holds
     std::mutex mu;
 
-    // process_device replays its launch sequence from a HIP graph while the
-    // call's arguments repeat (captured on the second call in a row with the
-    // same ones; last_key holds the last call's)
+    // process_device replays a launch sequence that one lane runs from a HIP
+    // graph while the call's arguments repeat (captured on the second call in a
+    // row with the same ones; last_key holds the last call's)
     struct GraphKey {
         const float *data, *ref;
         int64_t frame_stride, out_frame_stride;
@@ -277,7 +277,6 @@ struct Instance {
     hipGraphExec_t graph_exec = nullptr;
     GraphKey graph_key{}, last_key{};
     bool last_key_set = false;
-    bool captured = false, captured_forks = false;  // a graph was captured; one that forks lanes
     hipEvent_t fork_ev = nullptr, join_ev = nullptr;  // orders the instance stream with a null-stream caller
 
     // The host-buffer path (allocated on first use).  Requests overlap: a
@@ -1959,13 +1958,15 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
     // arguments; others, such as those of a caller that allocates its output
     // anew, are launched directly: capturing and instantiating costs more than
     // the few launches it would save once (64x48, one frame, a new output
-    // every call: 91 us with a capture each, 47 launched).  A sequence that
-    // forks lanes is captured only as the handle's first graph, and nothing
-    // after it: capturing one again with the graph before it destroyed has
-    // ended in a segmentation fault of the host whose cause is not known.
-    // Later arguments launch, which is no slower by much (8 frames of 640x360:
-    // one handle 231 us replayed, 201 launched; three handles in turn 227 and
-    // 238)
+    // every call: 91 us with a capture each, 47 launched).  Sequences that
+    // fork lanes are never captured: a capture after a graph of such a sequence
+    // was destroyed, this handle's or another's, has ended in a segmentation
+    // fault of the host whose cause is not known.  Launching them takes as long
+    // as replaying them did where several handles share the hardware queues,
+    // and less for one handle (us, replayed and launched, 8 frames: 64x48 167
+    // and 149, 640x360 231 and 201, 1280x720 349 and 322, 1920x1080 at
+    // block_step 4, bm_range 16 2398 and 2375; 640x360 by three handles in
+    // turn 227 and 228 to 238)
     const bool repeats = d.last_key_set && d.last_key == key;
     d.last_key = key;
     d.last_key_set = true;
@@ -1976,25 +1977,17 @@ int vsfeel_bm3d_process_device(vsfeel_bm3d *h, const vsfeel_bm3d_device_clip *cl
     // calls)
     std::fill(d.res_frame.begin(), d.res_frame.end(), -1);
     d.forget_sums();
-    const bool capturable = !d.captured || (!forks && !d.captured_forks);
-    if (d.graphs && !d.timing && count > 0 && (held || (repeats && capturable))) {
+    if (d.graphs && !d.timing && !forks && count > 0 && (held || repeats)) {
         // replay from a graph captured on the instance stream, ordered after
         // and before the caller's stream by events
         if (!held) {
             // the previous graph, or host-buffer requests, may still run on
             // the instance stream: capture on an idle one
             VSFEEL_HIP(hipStreamSynchronize(d.stream), "hipStreamSynchronize");
-            for (hipStream_t q : d.stream_l) {
-                if (q) {
-                    VSFEEL_HIP(hipStreamSynchronize(q), "hipStreamSynchronize");
-                }
-            }
             if (d.graph_exec) {
                 (void)hipGraphExecDestroy(d.graph_exec);
                 d.graph_exec = nullptr;
             }
-            d.captured = true;
-            d.captured_forks = forks;
             VSFEEL_HIP(hipStreamBeginCapture(d.stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
             const hipError_t e = enqueue(d.stream);
             hipGraph_t g = nullptr;

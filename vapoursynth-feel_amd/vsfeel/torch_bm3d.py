@@ -161,8 +161,8 @@ class Instance:
         _lib.load().vsfeel_bm3d_set_timing(self.handle, int(bool(enable)))
 
     def set_graphs(self, enable: bool) -> None:
-        """Replay process() from a captured HIP graph while its arguments repeat (default on at
-        radius 0; off at radius > 0, where direct launches overlap the two lanes better)."""
+        """Replay process() of one frame at radius 0 from a captured HIP graph while its arguments
+        repeat (the default there); calls on several lanes are always launched directly."""
         _lib.load().vsfeel_bm3d_set_graphs(self.handle, int(bool(enable)))
 
     def kernel_times(self) -> dict:
