@@ -2293,6 +2293,108 @@ __global__ __launch_bounds__(64) void bm3d_match_predictive(MatchArgs A)
     finish_group(A, G, blk, x, y, lane);
 }
 
+// The search of one block by one wavefront (no workgroup barrier).  cur_lds: 64
+// floats; for the temporal selection (t_rows > 0) a 64-entry stage of keys sk
+// and positions sxy, and t_rows distance rows of 2 ps_range + 1 floats, tdist
+template <int CM, bool EXACT>
+__device__ __forceinline__ void search_block(const MatchArgs &A, int blk, float *cur_lds, unsigned long long *sk,
+                                             uint32_t *sxy, float *tdist, int lane)
+{
+    const int by = blk / A.nx;
+    const int bx = blk - by * A.nx;
+    const int W = A.width, H = A.height, pitch = A.pitch, r = A.radius;
+    const int x = min(bx * A.step, W - 8);
+    const int y = min(by * A.step, H - 8);
+
+    const float *centre = A.plane[r];
+    // cur[c*8+i] = pixel (x+c, y+i), as the shader's cur[] (src/bm3d.comp:460-466)
+    cur_lds[lane] = centre[(long long)(y + (lane & 7)) * pitch + x + (lane >> 3)];
+    wave_lds_sync();
+    float cur_reg[EXACT ? 64 : 1];
+    if (EXACT) {
+#pragma unroll
+        for (int i = 0; i < 64; ++i) {
+            cur_reg[i] = cur_lds[i];
+        }
+    }
+
+    // spatial search (src/bm3d.comp:479-538)
+    TopList L;
+    list_reset(L);
+    if (A.spatial) {
+        // done by a kernel before this one
+        const uint2 e = A.spatial[(long long)blk * 8 + (lane & 7)];
+        if (lane < 8) {
+            L.key = uint64_t(e.x) << 32;
+            L.xy = e.y;
+        }
+    } else {
+        const int R = A.bm_range;
+        const int left = max(x - R, 0), right = min(x + R, W - 8);
+        const int top = max(y - R, 0), bottom = min(y + R, H - 8);
+        // the reference block's own row first: its candidates are usually
+        // among the best, so the top-8 threshold is tight from the start and
+        // few later candidates survive it (the result does not depend on the
+        // order: the list keeps the 8 smallest (distance, seq) keys)
+        const int rw = right - left + 1;
+        scan_window<CM, EXACT>(L, centre, pitch, H, cur_lds, cur_reg, left, right, y, y, (y - top) * rw, lane);
+        scan_window<CM, EXACT>(L, centre, pitch, H, cur_lds, cur_reg, left, right, top, bottom, 0, lane, y);
+    }
+    GroupList G;
+    G.e = __uint_as_float(uint32_t(L.key >> 32));
+    G.xy = L.xy;
+    G.z = r;
+
+    // temporal predictive search (src/bm3d.comp:540-637)
+    if (r > 0) {
+        const uint32_t spatial_xy = L.xy;
+        const int PR = A.ps_range;
+        const int win = (2 * PR + 1) * (2 * PR + 1);
+        for (int dir = -1; dir <= 1; dir += 2) {
+            uint32_t pred = spatial_xy;
+            for (int t = 1; t <= r; ++t) {
+                const int z = r + dir * t;
+                const float *plane = A.plane[z];
+                TopList F;
+                list_reset(F);
+                if (!EXACT && A.t_rows > 0) {
+                    // distance rows of the ps_num windows in this wavefront's
+                    // LDS, then one threshold selection
+                    const int wh = 2 * PR + 1;
+                    for (int i = 0; i < A.ps_num; ++i) {
+                        const uint32_t pxy = readlane_u32(pred, i);
+                        const int cx = int(pxy & 0xFFFFu), cyy = int(pxy >> 16);
+                        const int left = max(cx - PR, 0), right = min(cx + PR, W - 8);
+                        const int top = max(cyy - PR, 0), bottom = min(cyy + PR, H - 8);
+                        scan_window<CM, false, true>(F, plane, pitch, H, cur_lds, cur_reg, left, right, top,
+                                                     bottom, 0, lane, -1, tdist + i * wh * wh, wh);
+                    }
+                    wave_lds_sync();
+                    F = select_predictive(tdist, pred, A.ps_num, PR, W, H, sk, sxy, lane);
+                    wave_lds_sync();
+                } else {
+                    for (int i = 0; i < A.ps_num; ++i) {
+                        const uint32_t pxy = readlane_u32(pred, i);
+                        const int cx = int(pxy & 0xFFFFu), cyy = int(pxy >> 16);
+                        const int left = max(cx - PR, 0), right = min(cx + PR, W - 8);
+                        const int top = max(cyy - PR, 0), bottom = min(cyy + PR, H - 8);
+                        scan_window<CM, EXACT>(F, plane, pitch, H, cur_lds, cur_reg, left, right, top, bottom,
+                                               i * win, lane);
+                    }
+                }
+                for (int i = 0; i < A.ps_num; ++i) {
+                    const uint64_t fk = readlane_u64(F.key, i);
+                    const uint32_t fxy = readlane_u32(F.xy, i);
+                    group_insert(G, __uint_as_float(uint32_t(fk >> 32)), fxy, z, lane);
+                }
+                pred = F.xy;
+            }
+        }
+    }
+
+    finish_group(A, G, blk, x, y, lane);
+}
+
 // ---------------------------------------------------------------------------
 // Temporal predictive search of window sets too large for the kernel above
 // (ps_num windows of more than 32 rows together), one wavefront per ref block
@@ -2325,9 +2427,11 @@ __global__ __launch_bounds__(64) void bm3d_match_predictive(MatchArgs A)
 // D~ is off by the roundings of h and box, 2^-24 (2 box + N) < 2^-21 (N + D)
 // with N = sum_j |c_j|^2 + 8 |c7|^2; keys hold D~ + kStepEps N (never
 // negative).  The FP32 distance is off by less than 2^-20 D and what its
-// squares lose below 2^-126.  (box is infinite, and D~ with it, where N or D
-// is: `huge` blocks evaluate every candidate.)
+// squares lose below 2^-126.  (box is infinite, and D~ with it, where D is.)
 constexpr float kStepEps = 0x1p-20f, kStepRel = 0x1p-17f, kStepTiny = 0x1p-119f;
+// a block's self-distance one pixel away, over its |c|^2, from which on D~ is used
+// (2^-17: 8 margins; 2^-15 and 2^-13 took as long on every content measured)
+constexpr float kCoarse = 0x1p-17f;
 
 // LDS of one wavefront.  The strides spread a half wave's accesses over the
 // banks: rows (a lane per window row) as columns (one per lane, 8 of them).
@@ -2336,11 +2440,11 @@ struct StepLds {
     static constexpr int kWin = 64 / LW;       // windows at once
     static constexpr int kRows = LW + 6;       // of a window's source
     static constexpr int kWinStride = 8 * kRows;
+    float cur[64];                             // [column][row]
     double s[kWin * kWinStride];               // [window][7 columns][rows], then corr [window][8][rows]
     double d[7 * 8];                           // -2 (c_j - c7)
     double e[8];                               // |c_j|^2 - |c7|^2; e[7]: |c7|^2
     double none[LW];                           // NaN: corr of no candidate
-    float cur[64];                             // [column][row]
     uint32_t pos[64];                          // staged: row | k << 5 | window << 10
     unsigned long long key[32];
     uint32_t xy[32];
@@ -2367,8 +2471,8 @@ struct StepSearch {
     static __device__ __forceinline__ int sub_window(int lane) { return LW == 16 ? (lane >> 4) & 1 : 0; }
 
     __device__ __forceinline__ StepSearch(const MatchArgs &A, StepLds<LW> &lds, int lane)
-        : S(lds), W(A.width), H(A.height), PR(A.ps_range), PN(A.ps_num), wh(2 * PR + 1), npass(LW == 16 ? (PN + 1) >> 1 : PN), P(uint32_t(A.hb_pitch)),
-          HP4(uint32_t(A.hb_plane) * 4u),
+        : S(lds), W(A.width), H(A.height), PR(A.ps_range), PN(A.ps_num), wh(2 * PR + 1),
+          npass(LW == 16 ? (PN + 1) >> 1 : PN), P(uint32_t(A.hb_pitch)), HP4(uint32_t(A.hb_plane) * 4u),
           planes(__builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A.hb), 0,
                                                    uint32_t(3 * (2 * A.radius + 1)) * HP4, 0x00020000))
     {
@@ -2589,29 +2693,33 @@ __device__ __attribute__((noinline)) StepKeys steps_all(const __attribute__((add
     return {L.key, L.xy};
 }
 
+// bytes of a wavefront: StepLds, or the reference block and search_block's buffers
+template <int LW>
+__host__ __device__ inline int step_lds_bytes(int t_rows, int ps_range)
+{
+    const int general = 256 + 64 * 12 + 4 * t_rows * (2 * ps_range + 1), own = int(sizeof(StepLds<LW>));
+    return ((general > own ? general : own) + 15) & ~15;
+}
+
 template <int CM, int LW>
 __global__ __launch_bounds__(256, 4) void bm3d_match_steps(MatchArgs A)
 {
-    __shared__ StepLds<LW> lds_all[4];
+    extern __shared__ __align__(16) char slds[];
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     const int blk = xcd_block_id() * 4 + wave;
     if (blk >= A.nx * A.ny) {
         return;  // whole wavefront; no workgroup barrier follows
     }
-    StepLds<LW> &S = lds_all[wave];
+    char *const mem = slds + wave * step_lds_bytes<LW>(A.t_rows, A.ps_range);
+    StepLds<LW> &S = *reinterpret_cast<StepLds<LW> *>(mem);
     const int by = blk / A.nx, bx = blk - by * A.nx, r = A.radius;
     const int x = min(bx * A.step, A.width - 8), y = min(by * A.step, A.height - 8);
 
     // the reference block, its coefficients and norms
-    S.cur[lane] = A.plane[r][(long long)(y + (lane & 7)) * A.pitch + x + (lane >> 3)];
+    const float own = A.plane[r][(long long)(y + (lane & 7)) * A.pitch + x + (lane >> 3)];
+    S.cur[lane] = own;
     wave_lds_sync();
-    const StepSearch<CM, LW> T(A, S, lane);
-    const int PN = T.PN;
-    constexpr int kRowBits = T.kRowBits;
-    constexpr uint32_t pm = T.kPosMask;
-    // the smallest keys a lane keeps (one more is the bound of the rest)
-    constexpr int NK = 4;
     if (lane < 56) {
         S.d[lane] = -2.0 * (double(S.cur[lane]) - double(S.cur[56 + (lane & 7)]));
     }
@@ -2633,7 +2741,37 @@ __global__ __launch_bounds__(256, 4) void bm3d_match_steps(MatchArgs A)
     v += __uint_as_float(dpp_xor<1>(__float_as_uint(v), lane));
     v += __uint_as_float(dpp_xor<2>(__float_as_uint(v), lane));
     v += __uint_as_float(dpp_xor<4>(__float_as_uint(v), lane));
-    const bool huge = v > 1e28f || norm7 > 1e27;
+    // Content without noise (gradients, cartoons) has more near matches than D~
+    // tells apart.  The block's distance to itself one pixel to the right (e of
+    // lanes 0..31) or below (32..63), from its 56 pairs of pixels, stands for
+    // them: where it is not far above the resolution, or the pixels are huge or
+    // not finite, the general search takes the block.  (1280x720, block_step 4,
+    // 3 windows of 11 rows, us: three cartoons 375 to 392, all by the steps 782
+    // to 1155, by the general search's kernel 423 to 481; with noise from
+    // 0.4/255 on 202 and 314.  Radius 2, 4 windows of 17 rows, whose distances
+    // the general search offers to a list: cartoons 1590 to 2060, 3220 to
+    // 4810, 1360 to 1810; noise 735 and 1450.)  Blocks of equal pixels stay:
+    // most end at their first window's start.
+    {
+        const float dx = lane < 56 ? S.cur[min(lane + 8, 63)] - own : 0.0f;
+        const float dy = (lane & 7) < 7 ? S.cur[min(lane + 1, 63)] - own : 0.0f;
+        float e = (lane < 32 ? dx * dx : dy * dy) + __shfl_xor(lane < 32 ? dy * dy : dx * dx, 32);
+        e = row_sum16f(e, lane);
+        e += __shfl_xor(e, 16);
+        const bool clear = __ballot(e > v * kCoarse) == ~uint64_t(0), equal = __ballot(e != 0.0f) == 0;
+        if (!(v < 1e27f) || !(clear || equal)) {
+            unsigned long long *const sk = reinterpret_cast<unsigned long long *>(mem + 256);
+            search_block<CM, false>(A, blk, S.cur, sk, reinterpret_cast<uint32_t *>(sk + 64),
+                                    reinterpret_cast<float *>(sk + 96), lane);
+            return;
+        }
+    }
+    const StepSearch<CM, LW> T(A, S, lane);
+    const int PN = T.PN;
+    constexpr int kRowBits = T.kRowBits;
+    constexpr uint32_t pm = T.kPosMask;
+    // the smallest keys a lane keeps (one more is the bound of the rest)
+    constexpr int NK = 4;
     const float margin = (v + 8.0f * float(norm7)) * (1.0f + 0x1p-20f) * kStepEps + kStepTiny;
     const double base = __builtin_fma(8.0, norm7, double(margin));
     wave_lds_sync();
@@ -2747,7 +2885,7 @@ __global__ __launch_bounds__(256, 4) void bm3d_match_steps(MatchArgs A)
                     S.pos[half * 32 + at] = row | (uint32_t(T.column(ln)) << 5) | (w << 10);
                 }
             }
-            const uint64_t over = __ballot(huge || staged > 16 || m[NK] <= lim);
+            const uint64_t over = __ballot(staged > 16 || m[NK] <= lim);
             wave_lds_sync();
             const int most = max(__builtin_amdgcn_readlane(staged, 0), __builtin_amdgcn_readlane(staged, 32));
             for (int e0 = 0; e0 < min(most, 16); e0 += 4) {
@@ -2777,7 +2915,7 @@ __global__ __launch_bounds__(256, 4) void bm3d_match_steps(MatchArgs A)
             }
             for (int h = 0; h < 2; ++h) {
                 if (uint32_t(over >> (h * 32)) != 0u) {
-                    const uint32_t all = huge ? ~0u : uint32_t(__builtin_amdgcn_readlane(int(lim), h * 32));
+                    const uint32_t all = uint32_t(__builtin_amdgcn_readlane(int(lim), h * 32));
                     const StepKeys f = steps_all<CM, LW>(
                         (const __attribute__((address_space(4))) MatchArgs *)__builtin_amdgcn_kernarg_segment_ptr(),
                         (__attribute__((address_space(3))) StepLds<LW> *)&S, h, frame, all, pred, base);
@@ -2855,114 +2993,16 @@ template <int CM, bool EXACT>
 __global__ __launch_bounds__(256) void bm3d_match(MatchArgs A)
 {
     __shared__ float cur_all[4][64];
-    // temporal selection (t_rows > 0): per wavefront a 64-entry stage (keys,
-    // positions) and t_rows distance rows of 2 ps_range + 1 floats
     extern __shared__ __align__(16) unsigned long long tlds[];
     const int lane = lane_id();
     const int wave = threadIdx.x >> 6;
-
     const int blk = xcd_block_id() * 4 + wave;
-    const int nref = A.nx * A.ny;
-    if (blk >= nref) {
-        return;  // whole wavefront; no block-wide barrier follows
+    if (blk >= A.nx * A.ny) {
+        return;  // whole wavefront; no workgroup barrier follows
     }
-    const int by = blk / A.nx;
-    const int bx = blk - by * A.nx;
-    const int W = A.width, H = A.height, pitch = A.pitch, r = A.radius;
-    const int x = min(bx * A.step, W - 8);
-    const int y = min(by * A.step, H - 8);
-
-    const float *centre = A.plane[r];
-    float *cur_lds = cur_all[wave];
-    // cur[c*8+i] = pixel (x+c, y+i), as the shader's cur[] (src/bm3d.comp:460-466)
-    cur_lds[lane] = centre[(long long)(y + (lane & 7)) * pitch + x + (lane >> 3)];
-    wave_lds_sync();
-    float cur_reg[EXACT ? 64 : 1];
-    if (EXACT) {
-#pragma unroll
-        for (int i = 0; i < 64; ++i) {
-            cur_reg[i] = cur_lds[i];
-        }
-    }
-
-    // spatial search (src/bm3d.comp:479-538)
-    TopList L;
-    list_reset(L);
-    if (A.spatial) {
-        // done by bm3d_match_cols
-        const uint2 e = A.spatial[(long long)blk * 8 + (lane & 7)];
-        if (lane < 8) {
-            L.key = uint64_t(e.x) << 32;
-            L.xy = e.y;
-        }
-    } else {
-        const int R = A.bm_range;
-        const int left = max(x - R, 0), right = min(x + R, W - 8);
-        const int top = max(y - R, 0), bottom = min(y + R, H - 8);
-        // the reference block's own row first: its candidates are usually
-        // among the best, so the top-8 threshold is tight from the start and
-        // few later candidates survive it (the result does not depend on the
-        // order: the list keeps the 8 smallest (distance, seq) keys)
-        const int rw = right - left + 1;
-        scan_window<CM, EXACT>(L, centre, pitch, H, cur_lds, cur_reg, left, right, y, y, (y - top) * rw, lane);
-        scan_window<CM, EXACT>(L, centre, pitch, H, cur_lds, cur_reg, left, right, top, bottom, 0, lane, y);
-    }
-    GroupList G;
-    G.e = __uint_as_float(uint32_t(L.key >> 32));
-    G.xy = L.xy;
-    G.z = r;
-
-    // temporal predictive search (src/bm3d.comp:540-637)
-    if (r > 0) {
-        const uint32_t spatial_xy = L.xy;
-        const int PR = A.ps_range;
-        const int win = (2 * PR + 1) * (2 * PR + 1);
-        for (int dir = -1; dir <= 1; dir += 2) {
-            uint32_t pred = spatial_xy;
-            for (int t = 1; t <= r; ++t) {
-                const int z = r + dir * t;
-                const float *plane = A.plane[z];
-                TopList F;
-                list_reset(F);
-                if (!EXACT && A.t_rows > 0) {
-                    // distance rows of the ps_num windows in this wavefront's
-                    // LDS, then one threshold selection
-                    const int wh = 2 * PR + 1;
-                    unsigned long long *sk = tlds + wave * 64;
-                    uint32_t *sxy = reinterpret_cast<uint32_t *>(tlds + 256) + wave * 64;
-                    float *tdist = reinterpret_cast<float *>(tlds + 256 + 128) + wave * A.t_rows * wh;
-                    for (int i = 0; i < A.ps_num; ++i) {
-                        const uint32_t pxy = readlane_u32(pred, i);
-                        const int cx = int(pxy & 0xFFFFu), cyy = int(pxy >> 16);
-                        const int left = max(cx - PR, 0), right = min(cx + PR, W - 8);
-                        const int top = max(cyy - PR, 0), bottom = min(cyy + PR, H - 8);
-                        scan_window<CM, false, true>(F, plane, pitch, H, cur_lds, cur_reg, left, right, top,
-                                                     bottom, 0, lane, -1, tdist + i * wh * wh, wh);
-                    }
-                    wave_lds_sync();
-                    F = select_predictive(tdist, pred, A.ps_num, PR, W, H, sk, sxy, lane);
-                    wave_lds_sync();
-                } else {
-                    for (int i = 0; i < A.ps_num; ++i) {
-                        const uint32_t pxy = readlane_u32(pred, i);
-                        const int cx = int(pxy & 0xFFFFu), cyy = int(pxy >> 16);
-                        const int left = max(cx - PR, 0), right = min(cx + PR, W - 8);
-                        const int top = max(cyy - PR, 0), bottom = min(cyy + PR, H - 8);
-                        scan_window<CM, EXACT>(F, plane, pitch, H, cur_lds, cur_reg, left, right, top, bottom,
-                                               i * win, lane);
-                    }
-                }
-                for (int i = 0; i < A.ps_num; ++i) {
-                    const uint64_t fk = readlane_u64(F.key, i);
-                    const uint32_t fxy = readlane_u32(F.xy, i);
-                    group_insert(G, __uint_as_float(uint32_t(fk >> 32)), fxy, z, lane);
-                }
-                pred = F.xy;
-            }
-        }
-    }
-
-    finish_group(A, G, blk, x, y, lane);
+    search_block<CM, EXACT>(A, blk, cur_all[wave], tlds + wave * 64,
+                            reinterpret_cast<uint32_t *>(tlds + 256) + wave * 64,
+                            reinterpret_cast<float *>(tlds + 256 + 128) + wave * A.t_rows * (2 * A.ps_range + 1), lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -3880,14 +3920,16 @@ static hipError_t launch_temporal(const MatchArgs &a, int fp_mode, hipStream_t s
                           : go(bm3d_match_predictive<kFpExplicit, 0, 0>);
     }
     if (a.hb) {
-        auto go = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, grid, block, 0, s, a);
+        auto go = [&](auto kernel, int bytes) {
+            hipLaunchKernelGGL(kernel, grid, block, size_t(bytes) * 4, s, a);
             return hipGetLastError();
         };
         if (a.ps_range > 7) {
-            return fused ? go(bm3d_match_steps<kFpAll, 32>) : go(bm3d_match_steps<kFpExplicit, 32>);
+            const int bytes = step_lds_bytes<32>(a.t_rows, a.ps_range);
+            return fused ? go(bm3d_match_steps<kFpAll, 32>, bytes) : go(bm3d_match_steps<kFpExplicit, 32>, bytes);
         }
-        return fused ? go(bm3d_match_steps<kFpAll, 16>) : go(bm3d_match_steps<kFpExplicit, 16>);
+        const int bytes = step_lds_bytes<16>(a.t_rows, a.ps_range);
+        return fused ? go(bm3d_match_steps<kFpAll, 16>, bytes) : go(bm3d_match_steps<kFpExplicit, 16>, bytes);
     }
     const size_t tlds = size_t(temporal_lds_bytes(a.t_rows, a.ps_range));
     if (fused) {
