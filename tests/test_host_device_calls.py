@@ -128,3 +128,39 @@ def test_no_room_for_the_sums_leaves_the_search_without_them(calls):
         assert sums(tight) == (limit >= needed + planes)
         assert any("bm3d_match" in line for line in tight[1]["log"])
         assert tight[2]["live"] == 0
+
+
+def _bins(result):
+    assert result["rc"] == 0, result
+    return any("bm3d_gather" in line for line in result["log"])
+
+
+# 8 insertions and more, or 4 to 7 where blocks lie close together on frames of many blocks
+@pytest.mark.parametrize("w,h,kw,binned", [
+    (640, 360, dict(block_step=8, radius=2, ps_num=2), True),
+    (640, 360, dict(block_step=4, radius=1, ps_num=3), False),
+    (768, 720, dict(block_step=3, radius=1, ps_num=2), True),
+    (768, 720, dict(block_step=4, radius=1, ps_num=2), False),
+    (1920, 1080, dict(block_step=4, radius=1, ps_num=2), True),
+    (1920, 1080, dict(block_step=4, radius=1, ps_num=2, bm_range=20), False),
+    (1920, 1080, dict(block_step=4, radius=2, ps_num=1), False),
+    (1920, 1080, dict(block_step=5, radius=1, ps_num=3), False),
+    (3840, 2160, dict(block_step=8, radius=1, ps_num=2), False),
+])
+def test_which_calls_bin(calls, w, h, kw, binned):
+    kw = dict(dict(sigma=3.0, bm_range=9, ps_range=4), **kw)
+    assert _bins(calls([["create", w, h, 2, kw], ["process", "A", 0, 1]], lanes=1)[1]) == binned
+
+
+def test_bins_hold_what_dense_blocks_send(calls):
+    # (lists of 512 blocks overflowed at block_step 2 and 3, which was slower than no binning at all)
+    w, h, step = 512, 512, 2
+    live = {}
+    for ps_num in (2, 3, 4):
+        kw = dict(sigma=3.0, block_step=step, bm_range=7, radius=1, ps_num=ps_num, ps_range=3)
+        result = calls([["create", w, h, 2, kw], ["process", "A", 0, 2]])
+        assert _bins(result[1])
+        live[ps_num] = result[0]["live"]
+    # 2 lanes, 2 other frames, 16 x 16 cells, 8 bytes a block: 1024 blocks a cell, then 2048 and 2048
+    assert live[3] - live[2] == 2 * 2 * 16 * 16 * 8 * 1024
+    assert live[4] == live[3]

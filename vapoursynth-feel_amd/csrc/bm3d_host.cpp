@@ -1372,22 +1372,25 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
             hipSuccess) {
             return dev_fail(e, "hipMemcpy");
         }
+        // Binning pays where a group takes at least 8 temporal insertions.  With
+        // 4 to 7 it does on frames of many blocks, whose atomics' traffic
+        // outweighs the gather's pass over the frame, that lie close together:
+        // then every pixel takes many other-frame blocks, whatever the motion
+        // (a call's time with atomics over that with bins, least and most of
+        // noisy, letterboxed and clean clips: block_step 2 1.05 and 1.43, 3 0.98
+        // and 1.34, 4 0.94 and 1.30, 5 0.97 and 1.16, 6 0.94 and 1.06, 8 0.88
+        // and 1.07).  At block_step 4 the clips that lose most have less than
+        // about 100 k blocks (768x720, 1280x720: 0.96), bm_range 20 (0.95), the
+        // final pass (0.94) or radius 2 at ps_num 1 (0.96); the others make
+        // 0.98 to 1.30 at bm_range 5 to 12 and 0.96 to 1.15 at 16.
         const int insertions = 2 * d.radius * d.ps_num;
-        if (insertions >= 8 || (insertions >= 4 && d.nref >= 128 * kComputeUnits)) {
-            // binning pays where a group takes at least 8 temporal
-            // insertions, with 4 to 7 on frames of many blocks, where the
-            // gather's time is no longer its launch and the atomics' is their
-            // traffic (radius 1, ps_num 2: 3840x2160, block_step 4, estimate
-            // 973 us with atomics, 648 and a gather of 150 without, the frame
-            // 3.0 ms and 2.8; 825x532, 27 k blocks, 64 us, 43 and 17;
-            // 1280x720, block_step 8, 14 k, 53 us, 48 and 14).  How much
-            // depends on the motion, which decides how many of the blocks
-            // come from other frames: seven 3840x2160 clips moving by
-            // different parts of a pixel, 4 frames: 12.0 -> 10.7, 12.0 ->
-            // 10.8, 11.9 -> 11.3 ms, four with few such blocks 2 to 3 %
-            // slower.  A group holds at most 7 other-frame blocks (the self
-            // block is always a member); binning is skipped where its records
-            // would take more than 4 GiB, or find no room
+        const bool dense = d.block_step <= 3 ? d.nref >= 128 * kComputeUnits
+                                             : d.block_step == 4 && d.radius == 1 && !d.final_pass &&
+                                                   d.bm_range <= 16 && d.nref >= 384 * kComputeUnits;
+        if (insertions >= 8 || (insertions >= 4 && dense)) {
+            // A group holds at most 7 other-frame blocks (the self block is
+            // always a member); binning is skipped where its records would
+            // take more than 4 GiB, or find no room
             const long long tiles = (long long)d.tiles_x * d.tiles_y;
             const long long per_tile = (long long)d.tile_bx * d.tile_by * 7;
             const long long rec_bytes = tiles * per_tile * 256;
@@ -1406,7 +1409,17 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
                 d.rec_per_tile = int(per_tile);
                 d.cells_x = cx;
                 d.ncells = cx * cy;
+                // the blocks of all groups that may reach into a cell, were each
+                // group's from this frame ps_num, and a third more: blocks
+                // past a full list go down the atomic path after their records
+                // were written (1280x720, block_step 2, radius 1, ps_num 4, 4
+                // frames: 15.3 ms with lists of 512, 9.3 of 1024, 5.4 of 2048
+                // and of 4096, 8.1 with atomics alone)
+                const int reach = (cw + 7) * (cw + 7) / (d.block_step * d.block_step) * std::min(d.ps_num, 7);
                 d.cell_cap = 512;
+                while (d.cell_cap < 8192 && d.cell_cap * 3 < reach * 4) {
+                    d.cell_cap *= 2;
+                }
                 if (const char *cap = std::getenv("VSFEEL_BM3D_CELL_CAP")) {
                     // (tests: a small capacity sends most blocks down the atomic fallback)
                     d.cell_cap = std::min(std::max(std::atoi(cap), 1), 4096);
