@@ -164,3 +164,19 @@ def test_bins_hold_what_dense_blocks_send(calls):
     # 2 lanes, 2 other frames, 16 x 16 cells, 8 bytes a block: 1024 blocks a cell, then 2048 and 2048
     assert live[3] - live[2] == 2 * 2 * 16 * 16 * 8 * 1024
     assert live[4] == live[3]
+
+
+# the frames of the GPU tests of either kernel, and the line between them (32768 blocks, 64 x 44 pixels)
+@pytest.mark.parametrize("w,h,bm_range,block_step,kernel", [
+    (769, 727, 16, 4, "bm3d_match_cols"), (8203, 71, 16, 4, "bm3d_match_cols"), (93, 6301, 16, 4, "bm3d_match_cols"),
+    (64, 9000, 16, 4, "bm3d_match_cols"), (13202, 44, 16, 4, "bm3d_match_cols"),
+    (481, 275, 16, 4, "bm3d_match_rows"), (64, 40, 16, 4, "bm3d_match_rows"), (13202, 43, 16, 4, "bm3d_match_rows"),
+    (769, 727, 15, 4, "bm3d_match_rows"), (1920, 1080, 16, 5, "bm3d_match_rows"),
+])
+@pytest.mark.parametrize("radius", [0, 1])
+def test_which_kernel_searches(calls, w, h, bm_range, block_step, kernel, radius):
+    kw = dict(sigma=3.0, block_step=block_step, bm_range=bm_range, radius=radius)
+    result = calls([["create", w, h, 2, kw], ["process", "A", 0, 1]], lanes=1)[1]
+    assert result["rc"] == 0
+    spatial = {name for name in ("bm3d_match_cols", "bm3d_match_rows") if any(name in x for x in result["log"])}
+    assert spatial == {kernel}
