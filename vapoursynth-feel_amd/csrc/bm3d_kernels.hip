@@ -1858,14 +1858,16 @@ __global__ __launch_bounds__(256, 3) void bm3d_match_cols(MatchArgs A)
     // non-finite pixels): the distances themselves, a window row per thread,
     // as the sliding scan makes them (scan_row_sliding), from the source
     // region once more, column-major; top-8 from the rows' keys (select16,
-    // select_wave).  xblk blocks of a grid row at a time.
+    // select_wave).  xblk blocks at a time, of both grid rows where these have
+    // whole windows (few blocks of each are left then, usually: 1920x1080, dark
+    // noise clipped at 0, 398 us, a grid row at a time 435; a cartoon 269 and 296).
     const int CS = G.rrows | 1, DC = N, RHX = N;
     uint32_t *const xstage = reinterpret_cast<uint32_t *>(clds + L.h);       // [4][64] staged positions
     float *const region = reinterpret_cast<float *>(xstage + 256);           // [rcols][CS]
     uint32_t *const rowtop = reinterpret_cast<uint32_t *>(region + G.rcols * CS);  // [xblk][RHX][3]
     uint16_t *const dist = reinterpret_cast<uint16_t *>(rowtop + L.xblk * RHX * 3);  // [xblk][RHX][DC]
-    int *const list = reinterpret_cast<int *>(stage0);                       // [NB] blocks left, then their threshold
-    uint32_t *const xthr = reinterpret_cast<uint32_t *>(list + NB);
+    int *const list = reinterpret_cast<int *>(stage0);                       // [blocks] left, then their threshold
+    uint32_t *const xthr = reinterpret_cast<uint32_t *>(list + NB * VBC);
     const uint32_t pm = pos_mask(DC);
     for (int c0 = 0; c0 < ncols; c0 += 64) {
         const int c = c0 + lane;
@@ -1875,16 +1877,18 @@ __global__ __launch_bounds__(256, 3) void bm3d_match_cols(MatchArgs A)
             }
         }
     }
-    for (int v = 0; v < nv; ++v) {
-        const int y = min((by0 + v) * s, H - 8);
-        const int top = max(y - R, 0), rh = min(y + R, H - 8) - top + 1;
+    const int vstep = pair ? nv : 1;
+    auto row_of = [&](int bl) { return min((by0 + bl / NB) * s, H - 8); };
+    for (int v0 = 0; v0 < nv; v0 += vstep) {
+        const int rh = min(row_of(v0 * NB) + R, H - 8) - max(row_of(v0 * NB) - R, 0) + 1;
         __syncthreads();
         int left_over = 0;
         if (wave == 0) {
-            const bool in = lane < nb && over[v * NB + lane] != 0;
+            const int bl = v0 * NB + lane;
+            const bool in = lane < NB * vstep && bl % NB < nb && over[bl] != 0;
             const uint64_t mask = __ballot(in);
             if (in) {
-                list[__builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0)] = lane;
+                list[__builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0)] = bl;
             }
             left_over = __popcll(mask);
             if (lane == 0) {
@@ -1897,7 +1901,8 @@ __global__ __launch_bounds__(256, 3) void bm3d_match_cols(MatchArgs A)
             const int nq = min(L.xblk, left_over - q0);
             for (int i = t; i < nq * rh; i += 256) {
                 const int q = div_small(i, 1.0f / float(rh)), r = i - q * rh;
-                const int xb = min((bx0 + list[q0 + q]) * s, W - 8);
+                const int bl = list[q0 + q];
+                const int xb = min((bx0 + bl % NB) * s, W - 8), y = row_of(bl), top = max(y - R, 0);
                 const int left = max(xb - R, 0), right = min(xb + R, W - 8);
                 const float *cb = region + (xb - rx0) * CS + (y - ry0);
                 const uint3 t3 =
@@ -1913,7 +1918,8 @@ __global__ __launch_bounds__(256, 3) void bm3d_match_cols(MatchArgs A)
                 const int q = b0 + (lane >> 4);
                 const bool act = q < nq;
                 const int qs = act ? q : 0;
-                const int bx = bx0 + list[q0 + qs], xb = min(bx * s, W - 8);
+                const int bl = list[q0 + qs], bx = bx0 + bl % NB, by = by0 + bl / NB;
+                const int xb = min(bx * s, W - 8), y = row_of(bl), top = max(y - R, 0);
                 const int left = max(xb - R, 0), right = min(xb + R, W - 8);
                 const SpatialRows<CM> geo{right - left + 1, left, top, region + (xb - rx0) * CS + (y - ry0),
                                           region + (left - rx0) * CS + (top - ry0), CS};
@@ -1924,32 +1930,32 @@ __global__ __launch_bounds__(256, 3) void bm3d_match_cols(MatchArgs A)
                 if (act && staged <= 16) {
                     if (A.spatial) {
                         if (sub < 8) {
-                            A.spatial[(long long)((by0 + v) * A.nx + bx) * 8 + sub] =
+                            A.spatial[(long long)(by * A.nx + bx) * 8 + sub] =
                                 make_uint2(uint32_t(key >> 32), kxy);
                         }
                     } else {
-                        finish_group16(A, __uint_as_float(uint32_t(key >> 32)), kxy, (by0 + v) * A.nx + bx, xb, y,
-                                       sub);
+                        finish_group16(A, __uint_as_float(uint32_t(key >> 32)), kxy, by * A.nx + bx, xb, y, sub);
                     }
                 }
                 if (act && sub == 0) {
                     xthr[q] = staged > 16 ? thr : ~0u;
-                    over[v * NB + list[q0 + q]] = staged > 16 ? 1 : 0;
+                    over[bl] = staged > 16 ? 1 : 0;
                 }
             }
             __syncthreads();
             for (int q = wave; q < nq; q += 4) {
-                if (over[v * NB + list[q0 + q]] == 0) {
+                const int bl = list[q0 + q], bx = bx0 + bl % NB, by = by0 + bl / NB;
+                if (over[bl] == 0) {
                     continue;
                 }
-                const int bx = bx0 + list[q0 + q], xb = min(bx * s, W - 8);
+                const int xb = min(bx * s, W - 8), y = row_of(bl), top = max(y - R, 0);
                 const int left = max(xb - R, 0), right = min(xb + R, W - 8);
                 const SpatialRows<CM> geo{right - left + 1, left, top, region + (xb - rx0) * CS + (y - ry0),
                                           region + (left - rx0) * CS + (top - ry0), CS};
                 TopList T;
                 select_wave(rowtop + q * RHX * 3, dist + q * RHX * DC, DC, rh, geo, xthr[q], pm, lane,
                             xstage + wave * 64, T);
-                write_list(A, T, (by0 + v) * A.nx + bx, xb, y, lane);
+                write_list(A, T, by * A.nx + bx, xb, y, lane);
             }
             __syncthreads();
         }
