@@ -141,10 +141,14 @@ def _bins(result):
     (640, 360, dict(block_step=4, radius=1, ps_num=3), False),
     (768, 720, dict(block_step=3, radius=1, ps_num=2), True),
     (768, 720, dict(block_step=4, radius=1, ps_num=2), False),
-    (1920, 1080, dict(block_step=4, radius=1, ps_num=2), True),
+    (1280, 720, dict(block_step=4, radius=1, ps_num=2, bm_range=12), True),
+    (1280, 720, dict(block_step=4, radius=1, ps_num=2, bm_range=16), False),
+    (1920, 1080, dict(block_step=4, radius=1, ps_num=2, bm_range=16), True),
     (1920, 1080, dict(block_step=4, radius=1, ps_num=2, bm_range=20), False),
     (1920, 1080, dict(block_step=4, radius=2, ps_num=1), False),
     (1920, 1080, dict(block_step=5, radius=1, ps_num=3), False),
+    (2560, 1440, dict(block_step=5, radius=1, ps_num=2), True),
+    (2560, 1440, dict(block_step=5, radius=2, ps_num=1), False),
     (3840, 2160, dict(block_step=8, radius=1, ps_num=2), False),
 ])
 def test_which_calls_bin(calls, w, h, kw, binned):

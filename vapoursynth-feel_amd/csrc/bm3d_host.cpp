@@ -1378,15 +1378,21 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
         // then every pixel takes many other-frame blocks, whatever the motion
         // (a call's time with atomics over that with bins, least and most of
         // noisy, letterboxed and clean clips: block_step 2 1.05 and 1.43, 3 0.98
-        // and 1.34, 4 0.94 and 1.30, 5 0.97 and 1.16, 6 0.94 and 1.06, 8 0.88
-        // and 1.07).  At block_step 4 the clips that lose most have less than
-        // about 100 k blocks (768x720, 1280x720: 0.96), bm_range 20 (0.95), the
-        // final pass (0.94) or radius 2 at ps_num 1 (0.96); the others make
-        // 0.98 to 1.30 at bm_range 5 to 12 and 0.96 to 1.15 at 16.
-        const int insertions = 2 * d.radius * d.ps_num;
-        const bool dense = d.block_step <= 3 ? d.nref >= 128 * kComputeUnits
-                                             : d.block_step == 4 && d.radius == 1 && !d.final_pass &&
-                                                   d.bm_range <= 16 && d.nref >= 384 * kComputeUnits;
+        // and 1.34, 6 0.94 and 1.06, 8 0.88 and 1.07).  Between these it depends
+        // on the number of blocks and on bm_range, with which the tiles grow:
+        // block_step 4, bm_range 5 to 12, 34 k blocks 0.98 and 1.12, 57 k and
+        // more 0.97 and 1.30; bm_range 16, 57 k 0.96 and 1.09, 129 k and more
+        // 0.96 and 1.15 (of calls that the column search makes shorter); 20 0.95
+        // and 1.04; block_step 5, 83 k 0.97 and 1.08, 147 k and more 1.00 and
+        // 1.16; at block_step 4 the final pass 0.94 and 1.05, radius 2 at
+        // ps_num 1 0.96 and 1.08
+        const int insertions = 2 * d.radius * d.ps_num, r = d.bm_range;
+        const int few_from = d.block_step <= 3                ? 128
+                             : d.radius > 1 || d.final_pass   ? 0
+                             : d.block_step == 4 && r <= 16   ? (r <= 12 ? 192 : 384)
+                             : d.block_step == 5 && r <= 12   ? 512
+                                                              : 0;  // (blocks per compute unit; 0: never)
+        const bool dense = few_from > 0 && d.nref >= few_from * kComputeUnits;
         if (insertions >= 8 || (insertions >= 4 && dense)) {
             // A group holds at most 7 other-frame blocks (the self block is
             // always a member); binning is skipped where its records would
