@@ -93,7 +93,7 @@ def test_no_room_for_the_bins_leaves_the_atomic_scatter(calls, w, h, kw):
     assert roomy[0]["rc"] == roomy[1]["rc"] == 0 and bins(roomy)
     everything = roomy[0]["live"]
     # the records of a lane: 64 floats for each of 7 blocks of every group
-    ny, nx = (h - 8 + kw["block_step"] - 1) // kw["block_step"] + 1, (w - 8 + kw["block_step"] - 1) // kw["block_step"] + 1
+    ny, nx = ((q - 8 + kw["block_step"] - 1) // kw["block_step"] + 1 for q in (h, w))
     records = nx * ny * 7 * 64 * 4
     assert everything > 2 * records
     for limit in (everything - 1, everything - records, everything - records - 1, everything - 2 * records):
@@ -184,3 +184,21 @@ def test_which_kernel_searches(calls, w, h, bm_range, block_step, kernel, radius
     assert result["rc"] == 0
     spatial = {name for name in ("bm3d_match_cols", "bm3d_match_rows") if any(name in x for x in result["log"])}
     assert spatial == {kernel}
+
+
+# window sets of more than 32 rows (or wider than 25 columns), from 2048 blocks on, but not where 5 windows and more
+# overlap widely, or on small frames
+@pytest.mark.parametrize("w,h,block_step,ps_num,ps_range,kernel", [
+    (101, 97, 2, 3, 7, "bm3d_match_steps"), (101, 97, 2, 8, 4, "bm3d_match_steps"),
+    (101, 97, 2, 2, 8, "bm3d_match_steps"), (101, 97, 2, 1, 15, "bm3d_match_steps"),
+    (101, 97, 2, 8, 7, "bm3d_match_steps"), (101, 97, 2, 8, 15, "bm3d_match_steps"),
+    (101, 97, 2, 8, 8, "bm3d_matchI"), (101, 97, 2, 5, 12, "bm3d_matchI"), (101, 97, 2, 7, 4, "bm3d_matchI"),
+    (1280, 720, 8, 7, 4, "bm3d_match_steps"), (101, 97, 2, 3, 16, "bm3d_matchI"), (91, 89, 2, 3, 7, "bm3d_matchI"),
+    (101, 97, 2, 2, 7, "bm3d_match_predictive"), (101, 97, 2, 3, 4, "bm3d_match_predictive"),
+])
+def test_which_kernel_searches_the_other_frames(calls, w, h, block_step, ps_num, ps_range, kernel):
+    kw = dict(sigma=3.0, block_step=block_step, bm_range=5, radius=1, ps_num=ps_num, ps_range=ps_range)
+    result = calls([["create", w, h, 3, kw], ["process", "A", 0, 1]], lanes=1)[1]
+    assert result["rc"] == 0
+    names = ("bm3d_match_steps", "bm3d_match_predictive", "bm3d_matchI")  # (the last: bm3d_match<..>, mangled)
+    assert {name for name in names if any(name in line for line in result["log"])} == {kernel}

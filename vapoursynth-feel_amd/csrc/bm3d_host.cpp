@@ -1167,12 +1167,25 @@ std::string parse_args(const vsfeel_bm3d_args &a, Instance &d)
             // for every SIMD on (283x280, 4900 blocks, 2 windows of 17 rows:
             // 35 us against the general search's 43; 341x230, 1218 blocks, 4
             // of 15: 32 against 40, but 6 us more for the launch of the sums;
-            // 166x114, 408 blocks, 2 of 17: 36 against 28); a lane addresses
+            // 166x114, 408 blocks, 2 of 17: 36 against 28).  Five windows and
+            // more overlap, so that many candidates tie with themselves: where
+            // a window's columns leave many of its 32 lanes idle besides, the
+            // second walks that this costs take more than is won (a call's time
+            // with the general search over that with this one, noisy clips,
+            // 1280x720, block_step 8: 5 to 8 windows of 21 and 25 rows 0.69 to
+            // 1.25, of 17 rows 1.05 to 1.25 and at 400x300 0.89 to 1.04; of 11
+            // to 15 rows, 16 lanes a window, 1.2 to 1.8, of 31 1.0 to 1.8), and
+            // small frames do not hide them where the general search has its
+            // distance rows (400x300, 4800 blocks, 5 to 7 of 9 rows: 0.87 to
+            // 0.99; 1280x720, 14 k: 0.99 to 1.17).  Clips without noise take
+            // 0.93 to 1.3 up to 64 rows, 0.73 to 0.89 beyond.  A lane addresses
             // all sums of its window's frames by 32-bit byte offsets
+            const bool many = d.ps_num >= 5;
+            const bool overlap = many && ((d.ps_range >= 8 && d.ps_range <= 12) || (rows <= 64 && d.nref < 48 * kComputeUnits));
             const int hp = (d.width + 15) & ~15;
             const long long plane = (long long)hp * (d.height + kSumPlanePad);
             if (d.radius <= 2 && !d.pred_pair && d.ps_range <= kStepsMaxRange && d.nref >= 8 * kComputeUnits &&
-                plane * 3 * d.tw * 4 < (1LL << 32)) {
+                !overlap && plane * 3 * d.tw * 4 < (1LL << 32)) {
                 d.hb_pitch = hp;
                 d.hb_plane = plane;
             }
