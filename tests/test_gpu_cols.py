@@ -1,9 +1,9 @@
-"""bm3d_match_cols (bm_range 16 at block_step 4) against the oracle: groups entry for entry.
+"""Spatial search at bm_range 16, block_step 4 on small frames against the oracle: groups entry for entry.
 
-The kernel's edges: frames of exactly its run's region, partly filled runs and
-grid-row pairs, windows clipped on every side; and the content its expanded
-distances do not resolve, which has to end in the exact distances: equal and
-near-equal pixels, huge and non-finite ones, texture along columns.
+bm3d_match_rows searches these; bm3d_match_cols takes frames of 32768 blocks
+and more (test_gpu_cols_content.py, test_gpu_cols_large.py).  Frames of a few
+runs, partly filled runs, windows clipped on every side; equal and near-equal
+pixels, huge and non-finite ones, texture along columns.
 """
 
 import os
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 NT = min(16, os.cpu_count() or 1)
 
-# 64 columns by 40 rows (one grid row per run); from about 480x272 on, runs of two grid rows
+# 135 to 8160 blocks
 SIZES = [(64, 40), (65, 45), (91, 77), (93, 131), (481, 275)]
 
 

@@ -1,11 +1,11 @@
 """Graph replay of the device entry point against direct launches.
 
-process() captures its launch sequence into a HIP graph on the first call
-with a given set of arguments and replays it afterwards.  Every replay, with
-the program's own eager work and synchronisations between replays, must give
-bit-identical frames to the directly launched sequence (the accumulation is
-integer fixed point, so the results are deterministic), also after the clip
-memory is rewritten in place and after the output moves.  Host-buffer
+process() with graphs switched on (which captures calls on one lane only;
+those here are on several) must give bit-identical frames to the directly
+launched sequence at every call (the accumulation is integer fixed point, so
+the results are deterministic), with the program's own eager work and
+synchronisations between calls, after the clip memory is rewritten in place
+and after the output moves.  Host-buffer
 requests (getFrame) with request graphs on launch from per-slot graphs
 updated per request, and must equal direct launches in any order and from
 several threads.

@@ -1142,10 +1142,11 @@ std::string parse_args(const vsfeel_bm3d_args &a, Instance &d)
         }
         // bm3d_match_cols where it was compiled, the frame holds its run's
         // region and there are blocks enough to hide the exact search of the
-        // runs without noise, which few blocks wait for (cartoon 428x316: 43
-        // us by rows, 61 by columns; 853x481, 25 k blocks: noisy 65 and 55,
-        // cartoon 78 and 84; 1280x720, 57 k: 128 and 97, 135 and 142;
-        // 1920x1080: 261 and 198, 284 and 261)
+        // runs without noise, which few blocks wait for (us by rows and by
+        // columns, cartoon 428x316: 43 and 61; 853x481, 25 k blocks: 78 and 84,
+        // noisy 65 and 55; calls of 6 frames, ms, cartoon 768x720, 34 k: 0.73
+        // and 0.69 to 0.74, noisy 0.71 and 0.62; 1280x720, 57 k: 1.10 and 1.03,
+        // 1.08 and 0.91; 1920x1080: 2.29 and 2.07, 2.20 and 1.88)
         const ColsGeometry g = cols_geometry(16, 4, 2);
         d.use_cols = d.run_blocks > 0 && d.bm_range == 16 && d.block_step == 4 && d.width >= g.rcols &&
                      d.height >= g.rrows && d.nref >= 128 * kComputeUnits;
@@ -1455,9 +1456,7 @@ int vsfeel_bm3d_create(const vsfeel_bm3d_args *args, vsfeel_bm3d **out, char *er
         if (!d.short_windows && max_lanes > 1) {
             // the lanes' own buffer sets (lane 0 has the instance's)
             d.lanes = std::min(d.radius == 0 ? Instance::kLanes : Instance::kTemporalLanes, max_lanes);
-            // at radius > 0 the replayed graph overlapped the lanes' cross-
-            // linked branches less than direct launches do (980 against 1024
-            // frames/s at 1080p radius 2): launch directly by default
+            // (calls on several lanes are never captured: process_device)
             d.graphs = d.radius == 0;
             if ((e = hipEventCreateWithFlags(&d.lane_fork, hipEventDisableTiming)) != hipSuccess) {
                 return dev_fail(e, "hipEventCreate");

@@ -27,8 +27,6 @@
 // which is what keeps distances, coefficients and thresholds bit-identical to
 // the CPU restatement of the reference shaders.
 
-#include <type_traits>
-
 #include "bm3d_device.hpp"
 
 namespace vsfeel {
@@ -752,12 +750,13 @@ __global__ __launch_bounds__(256) void bm3d_match_rows(MatchArgs A)
 // columns): lanes and row sets cut those clusters, so that the keys hold all
 // matches for all but a few blocks.
 //
-// Bound by VALU issue: 90 M wave instructions per 1080p frame (150 us of 195)
-// against bm3d_match_rows' 144 M; 53 KB of LDS, 3 workgroups per CU.  Two
+// Bound by VALU issue: 89 M wave instructions per 1080p frame (146 us of 189)
+// against bm3d_match_rows' 145 M; 53 KB of LDS, 3 workgroups per CU.  Two
 // grid rows per run share staging and sums (44 region rows instead of 80).
 // bm_range 16, block_step 4, 1920x1080, this kernel against bm3d_match_rows
 // (first passes, one lane): noisy images 0.195 / 0.251 ms, letterboxed 0.205
-// / 0.323, without noise 0.248 / 0.277, texture along columns 0.247 / 0.247.
+// / 0.323, without noise 0.242 / 0.277, texture along columns 0.247 / 0.247;
+// dark noise clipped at 0, whose blocks tie with the black ones, 0.398 / 0.353.
 // ---------------------------------------------------------------------------
 
 // |D~ - D| <= kEps (N + box) + kTiny for the candidate, where N = sum_j |c_j|^2
@@ -1425,7 +1424,7 @@ __global__ __launch_bounds__(256, 3) void bm3d_match_cols(MatchArgs A)
     // the keys' offset: first the term of each column j = 0..6, a thread per
     // block and column (j = 7: the constant of all later candidates), the
     // rows split over the workgroup.  Two grid rows 4 rows apart with whole
-    // windows share terms (walk_column_pair)
+    // windows share terms (walk_lane_pair)
     constexpr bool kPairs = s == 4 && VBC == 2;
     const bool pair = kPairs && nv == 2 && y_last == y_first + 4 && y_first >= R && y_last + R <= H - 8;
     if (!exact) {
@@ -2071,7 +2070,7 @@ __global__ __launch_bounds__(64) void bm3d_match_predictive(MatchArgs A)
 
     cur[lane] = A.plane[r][(long long)(y + (lane & 7)) * pitch + x + (lane >> 3)];
 
-    // the spatial top-8 (bm3d_match_cols) starts the group and predicts
+    // the spatial search's top-8 starts the group and predicts
     TopList L;
     list_reset(L);
     {
@@ -3708,7 +3707,7 @@ __global__ __launch_bounds__(256) void bm3d_tile_reduce(ReduceArgs A)
             wt += vw[k];
         }
     } else {
-        // many tiles over a pixel (small frames: up to all of them): 8 at a
+        // many tiles over a pixel (small frames: up to all of them): 12 at a
         // time, their origins and then their values loaded together, added
         // one by one in the tiles' order (52x54 at block_step 4, bm_range 20:
         // 50 us with a load waited for per tile, 28 now; 80x44 at 4, 20: 48 us
@@ -3983,10 +3982,11 @@ hipError_t launch_match(const MatchArgs &a, int fp_mode, hipStream_t s, bool tem
         }
         // bm_range 16 at block_step 4 (the benchmark harness) takes the
         // expanded distances, whose sums and selection cost the same for any
-        // window: worth it from about 1000 candidates on.  With run-time
-        // geometry they were slower (778x751, bm_range 12 at block_step 8:
-        // 43 us against 24), compiled for bm_range 9 not faster (640x360 at
-        // block_step 8: 18 against 17 us; 512x512 at 4: 23 against 27 us)
+        // window.  They are compiled for that pair alone: with run-time
+        // geometry they were slower (778x751, bm_range 12 at block_step 8: 43
+        // us against 24), compiled for bm_range 9 not faster (640x360 at
+        // block_step 8: 18 against 17 us; 512x512 at 4: 23 against 27 us, its
+        // call no faster); other wide windows were not measured
         if (a.use_cols) {
             auto cols = [&](auto kernel) {
                 const ColsGeometry g = cols_geometry(16, 4, 2);
